@@ -19,6 +19,7 @@
 #include "qmc_derivs.hpp"
 #include "qmc_device.hpp"
 #include "qmc_dmc.hpp"
+#include "qmc_group.hpp"
 #include "qmc_kernels.hpp"
 #include "qmc_noalloc.hpp"
 #include "qmc_refresh.hpp"
@@ -115,12 +116,16 @@ struct qmc_system {
   const EngineOps* ops = nullptr;      // register-engine kernels in use
   const EngineOps* ops_spec = nullptr; // compiled shell structure matching the system, if any
   const EngineOps* ops_gen = nullptr;  // generic kernels of the electron-count shape
+  const GroupOps* gops = nullptr;      // lane-group kernels in use (the same shapes and shell structures)
+  const GroupOps* gops_spec = nullptr;
+  const GroupOps* gops_gen = nullptr;
   const DerivOps* dops = nullptr;      // derivative kernels in use
   const DerivOps* dops_spec = nullptr; // specialised to the shell structure (may equal dops_gen)
   const DerivOps* dops_gen = nullptr;
   int32_t engine = QMC_ENGINE_AUTO;
   void pick_ops() {
     ops = (engine == QMC_ENGINE_GENERIC || !ops_spec) ? ops_gen : ops_spec;
+    gops = (engine == QMC_ENGINE_GENERIC || !gops_spec) ? gops_gen : gops_spec;
     dops = (engine == QMC_ENGINE_GENERIC || !dops_spec) ? dops_gen : dops_spec;
   }
   bool dirty = true;
@@ -450,6 +455,8 @@ int upload(qmc_system* s) {
   s->ops_spec = find_engine(*d64, false);
   if (s->ops_spec && !s->ops_spec->match) s->ops_spec = nullptr;
   s->ops_gen = find_engine(*d64, true);
+  s->gops_spec = find_group(*d64, false);
+  s->gops_gen = find_group(*d64, true);
   s->dops_spec = find_derivs(*d64, false);
   s->dops_gen = find_derivs(*d64, true);
   s->pick_ops();
@@ -1539,7 +1546,9 @@ int qmc_ensemble_sweeps(qmc_ensemble* e, const qmc_sweep_params* p, double* e_su
   const bool tdd = p->move == QMC_MOVE_DRIFT && s->tile_dd(e->prec);
   const int nblk = p->move == QMC_MOVE_SINGLE ? (int)sweep_blocks(e)
                    : tdd                       ? (int)tile_blocks(e->W)
-                                               : (int)(wave ? e->W : (e->W + 63) / 64);
+                   : wave                      ? (int)e->W
+                   : p->move == QMC_MOVE_ALL   ? (int)((e->W + s->gops->wpb - 1) / s->gops->wpb)
+                                               : (int)((e->W + 63) / 64);
   const int refresh = p->refresh_interval > 0 ? p->refresh_interval : 0;
   int chunk = p->steps_per_launch > 0 ? p->steps_per_launch : 16;
   if ((rc = ensure_cap(&e->partial, &e->partial_cap, (size_t)chunk * nblk * 3))) return rc;
@@ -1588,9 +1597,11 @@ int qmc_ensemble_sweeps(qmc_ensemble* e, const qmc_sweep_params* p, double* e_su
       else if (wave)
         HIP_TRY(wave_ae<float>(s->d64, s->d32, e->view<float>(), s->shape(), A, e->partial, trace, e->st));
       else if (e->prec == QMC_FP64)
-        HIP_TRY(s->ops->ae64(s->d64, s->d64, e->view<double>(), A, e->partial, trace, e->st));
+        HIP_TRY((s->no_series() ? s->gops->ae64_ns : s->gops->ae64)(s->d64, e->view<double>(), A, e->partial, trace,
+                                                                    e->st));
       else
-        HIP_TRY(s->ops->ae32(s->d64, s->d32, e->view<float>(), A, e->partial, trace, e->st));
+        HIP_TRY((s->no_series() ? s->gops->ae32_ns : s->gops->ae32)(s->d64, e->view<float>(), A, e->partial, trace,
+                                                                    e->st));
       e->inverse_stale = true;
     }
     if (e->timing) HIP_TRY(hipEventRecord(e->ev[2 * nl + 1], e->st));

@@ -75,86 +75,6 @@ __global__ void __launch_bounds__(64) dd_sweep_kernel(const DevSys<T>* __restric
 }
 
 // ---------------------------------------------------------------------------
-// all-electron Metropolis (MCMCSimulation::metropolis_step, vmc.rs:95-119):
-// every electron moved at once, full recomputation of ln|psi|, E_L
-// recomputed on acceptance only and cached otherwise.
-// ---------------------------------------------------------------------------
-template <int NU, int ND, class Bs, class T>
-__global__ void __launch_bounds__(64) all_electron_kernel(const DevSys<double>* __restrict__ Sd,
-                                                          const DevSys<T>* __restrict__ Sp, EnsView<T> E,
-                                                          SweepArgs A, double* __restrict__ partial,
-                                                          double* __restrict__ el_trace) {
-  const DevSys<T>& S = *Sp;
-  const int64_t w = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  const bool live = w < E.W;
-  const int64_t wl = live ? w : E.W - 1;
-  WalkerRegs<NU, ND, T> R, Q;
-  load_positions<NU, ND>(S, E.pos, E.ld, wl, R);
-  double ldet = E.logdet[wl], ju = E.ju[wl], sgn = E.sign[wl], el = E.eloc[wl];
-  const uint32_t k0 = (uint32_t)A.seed, k1 = (uint32_t)(A.seed >> 32);
-  const uint32_t wid = (uint32_t)(A.walker0 + wl);
-  const T sigma = (T)A.step_size;
-  const uint32_t N = (uint32_t)S.n_elec;
-  for (int s = 0; s < A.n_steps; ++s) {
-    const uint32_t step = A.step0 + (uint32_t)s;
-#pragma unroll
-    for (int k = 0; k < NU; ++k) {
-      T z[3];
-      Rng<T>::normals3(philox(wid, step, (uint32_t)S.sector_elec[0][k], RNG_ALL, k0, k1), z);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) Q.ru[k][c] = R.ru[k][c] + sigma * z[c];
-    }
-#pragma unroll
-    for (int k = 0; k < ND; ++k) {
-      T z[3];
-      Rng<T>::normals3(philox(wid, step, (uint32_t)S.sector_elec[1][k], RNG_ALL, k0, k1), z);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) Q.rd[k][c] = R.rd[k][c] + sigma * z[c];
-    }
-    double lu, su, ldn, sd;
-    sector_inverse<NU, T, Bs>(*Sd, 0, Q.ru, Q.au, lu, su);
-    sector_inverse<ND, T, Bs>(*Sd, 1, Q.rd, Q.ad, ldn, sd);
-    const double jun = jastrow_u<NU, ND, T, Bs>(*Sd, Q.ru, Q.rd);
-    const double U = u01d(philox(wid, step, N, RNG_ALL, k0, k1).x);
-    int acc = 0;
-    if (U < exp(2.0 * ((lu + ldn + jun) - (ldet + ju)))) {
-      // only the positions persist; the inverses serve this E_L and go
-#pragma unroll
-      for (int k = 0; k < NU; ++k)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) R.ru[k][c] = Q.ru[k][c];
-#pragma unroll
-      for (int k = 0; k < ND; ++k)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) R.rd[k][c] = Q.rd[k][c];
-      ldet = lu + ldn;
-      ju = jun;
-      sgn = su * sd;
-      el = local_energy<NU, ND, T, Bs>(S, Q.ru, Q.au, Q.rd, Q.ad, nullptr, nullptr, 0);
-      acc = 1;
-    }
-    if (el_trace && live) el_trace[(int64_t)s * A.trace_ld + w] = el;
-    double e1 = live ? el : 0.0, e2 = live ? el * el : 0.0, a = live ? (double)acc : 0.0;
-    e1 = wave_sum(e1);
-    e2 = wave_sum(e2);
-    a = wave_sum(a);
-    if (threadIdx.x == 0) {
-      double* p = partial + ((int64_t)s * gridDim.x + blockIdx.x) * 3;
-      p[0] = e1;
-      p[1] = e2;
-      p[2] = a;
-    }
-  }
-  if (live) {
-    store_positions<NU, ND>(S, E.pos, E.ld, w, R);
-    E.logdet[w] = ldet;
-    E.ju[w] = ju;
-    E.sign[w] = sgn;
-    E.eloc[w] = el;
-  }
-}
-
-// ---------------------------------------------------------------------------
 // batched per-configuration evaluation of the trait methods.  Input
 // positions are [W][N][3] FP64 in global electron order (the reference's
 // Vec<Vector3<f64>> layout); outputs are written walker-major.
@@ -264,12 +184,6 @@ struct Launch {
     dd_sweep_kernel<NU, ND, Bs, Js, T><<<nblocks(E.W), 64, 0, st>>>((const DevSys<T>*)St, E, A, partial, trace);
     return hipGetLastError();
   }
-  static hipError_t all_electron(const void* Sd, const void* St, EnsView<T> E, SweepArgs A, double* partial,
-                                 double* trace, hipStream_t st) {
-    all_electron_kernel<NU, ND, Bs, T><<<nblocks(E.W), 64, 0, st>>>((const DevSys<double>*)Sd,
-                                                                   (const DevSys<T>*)St, E, A, partial, trace);
-    return hipGetLastError();
-  }
   static hipError_t eval(const void* Sd, const void* St, int64_t W, const double* pos, EvalOut O, int* sing,
                          hipStream_t st) {
     eval_kernel<NU, ND, Bs, T><<<nblocks(W), 64, 0, st>>>((const DevSys<double>*)Sd, (const DevSys<T>*)St, W,
@@ -305,12 +219,6 @@ static EngineOps make_ops(const char* name, bool (*match)(const DevSys<double>&)
   o.sweep32 = &Launch<NU, ND, Bs, float>::template sweep<JsRt>;
   o.sweep64_ns = &Launch<NU, ND, Bs, double>::template sweep<JsFast>;
   o.sweep32_ns = &Launch<NU, ND, Bs32, float>::template sweep<JsFast>;
-  // All-electron moves always run the run-time-loop kernels: the CH4/STO-3G
-  // all-electron kernel specialised to its shell structure disagreed with
-  // them (and with the oracle) from the first step while every other
-  // specialised kernel agrees, and no cause has been found in the source.
-  o.ae64 = &Launch<NU, ND, RtBasis, double>::all_electron;
-  o.ae32 = &Launch<NU, ND, RtBasis, float>::all_electron;
   o.dd64 = &Launch<NU, ND, Bs, double>::template dd<JsRt>;
   o.dd32 = &Launch<NU, ND, Bs, float>::template dd<JsRt>;
   o.dd64_ns = &Launch<NU, ND, Bs, double>::template dd<JsFast>;
