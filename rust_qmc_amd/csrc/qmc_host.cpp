@@ -23,6 +23,7 @@
 #include "qmc_kernels.hpp"
 #include "qmc_noalloc.hpp"
 #include "qmc_refresh.hpp"
+#include "qmc_terms.hpp"
 #include "qmc_batch.hpp"
 #include "qmc_tile.hpp"
 #include "qmc_wave.hpp"
@@ -153,7 +154,12 @@ struct qmc_system {
   MoDerivPair* mdp = nullptr;
   MoDerivEntry* mde = nullptr;
   int mdp0[3] = {0, 0, 0};
+  TermTab* terms = nullptr;  // parameters of the one-electron-per-lane kernels, when they fit the system
+  bool terms_ok = false;
+  // evaluation and derivatives one electron per lane, unless the wave engine is selected
+  bool use_terms() const { return wave() && terms_ok && engine != QMC_ENGINE_WAVE; }
   ~qmc_system() {
+    if (terms) (void)hipFree(terms);
     if (d64) (void)hipFree(d64);
     if (d32) (void)hipFree(d32);
     if (mdp) (void)hipFree(mdp);
@@ -451,6 +457,12 @@ int upload(qmc_system* s) {
       HIP_TRY(hipMemcpy(s->mdp, pairs.data(), pairs.size() * sizeof(MoDerivPair), hipMemcpyHostToDevice));
       HIP_TRY(hipMemcpy(s->mde, ents.data(), ents.size() * sizeof(MoDerivEntry), hipMemcpyHostToDevice));
     }
+    auto tab = std::make_unique<TermTab>();
+    s->terms_ok = terms_table(*d64, pairs.data(), ents.data(), s->mdp0, *tab);
+    if (s->terms_ok) {
+      if (!s->terms) HIP_TRY(hipMalloc(&s->terms, sizeof(TermTab)));
+      HIP_TRY(hipMemcpy(s->terms, tab.get(), sizeof(TermTab), hipMemcpyHostToDevice));
+    }
   }
   s->ops_spec = find_engine(*d64, false);
   if (s->ops_spec && !s->ops_spec->match) s->ops_spec = nullptr;
@@ -551,10 +563,16 @@ int need_engine(const qmc_system* s) {
   return QMC_OK;
 }
 
-// The derivative matrix Y of A.W walkers in the arithmetic type prec: the
-// wave derivative kernel when the wave or tile engine runs the system (or
+// The derivative matrix Y of A.W walkers in the arithmetic type prec (FP64
+// in the one-electron-per-lane kernel, which serves both precisions): that
+// kernel for the 21 + 21-electron systems it fits, else the wave derivative
+// kernel when the wave or tile engine runs the system (or
 // its MO coefficients follow the geometry), else the register kernels.
 int launch_derivs(const qmc_system* s, DerivArgs A, int32_t prec, hipStream_t st) {
+  if (s->use_terms()) {
+    HIP_TRY(terms_derivs(s->d64, s->terms, A, st));
+    return QMC_OK;
+  }
   if (s->wave() || !s->dops || s->h.mo_rule != QMC_MO_FIXED) {
     if (int rc = need_engine(s)) return rc;
     if (s->h.n_elec() > 64) return fail(QMC_ERR_UNSUPPORTED, "the wave derivative kernel takes up to 64 electrons");
@@ -1168,7 +1186,9 @@ int qmc_evaluate(const qmc_system* sys, int64_t W, const double* pos, double* lo
   std::unique_ptr<int, void (*)(int*)> sing_guard(sing, [](int* p) { (void)hipFree(p); });
   HIP_TRY(hipMemsetAsync(sing, 0, sizeof(int), st));
   EvalOut O{(double*)L.dev, (double*)S.dev, (double*)G.dev, (double*)Lp.dev, (double*)E.dev};
-  if (sys->wave()) {
+  if (sys->use_terms()) {
+    HIP_TRY(terms_eval(sys->d64, sys->terms, W, (const double*)P.dev, O, sing, st));
+  } else if (sys->wave()) {
     if (sys->precision == QMC_FP64)
       HIP_TRY(wave_eval<double>(sys->d64, sys->d64, W, (const double*)P.dev, sys->shape(), O, sing, st));
     else
