@@ -34,20 +34,20 @@ struct TermLds {
 // radial sums of a shell: R = sum c e, and with DER R_a = sum c a e and
 // R_aa = sum c a^2 e
 template <int NP, bool P, bool DER>
-__device__ __forceinline__ void radial(const TermShell& q, double r2, double s[3], double p[3]) {
+__device__ __forceinline__ void radial(const TermPrim* q, double r2, double s[3], double p[3]) {
 #pragma unroll
   for (int k = 0; k < 3; ++k) s[k] = p[k] = 0.0;
 #pragma unroll
   for (int k = 0; k < NP; ++k) {
-    const double a = q.ex[k], e = M<double>::exn(-a * r2);
-    const double cs = q.cs[k] * e;
+    const double a = q[k].ex, e = M<double>::exn(-a * r2);
+    const double cs = q[k].cs * e;
     s[0] += cs;
     if constexpr (DER) {
       s[1] += cs * a;
       s[2] += cs * a * a;
     }
     if constexpr (P) {
-      const double cp = q.cp[k] * e;
+      const double cp = q[k].cp * e;
       p[0] += cp;
       if constexpr (DER) {
         p[1] += cp * a;
@@ -68,12 +68,10 @@ __device__ __forceinline__ void by_count(int np, F f) {
     f(std::integral_constant<int, 6>{});
 }
 
-// sums over the 21 electrons of each walker of NR (at most 21) values per
-// lane, through this wavefront's row buffer: out[r][g]
+// sums over the 21 electrons of each walker of the NR (at most 20) values
+// per lane that this wavefront stored at buf[r * 64 + lane]: out[r][g]
 template <int NR>
-__device__ __forceinline__ void lane_sums(double* buf, int lane, const double* v, double (*out)[GW]) {
-#pragma unroll
-  for (int r = 0; r < NR; ++r) buf[r * 64 + lane] = v[r];
+__device__ __forceinline__ void lane_sums(const double* buf, int lane, double (*out)[GW]) {
   wave_sync();
   for (int t = lane; t < NR * GW; t += 64) {
     const int r = t / GW, g = t % GW;
@@ -83,6 +81,12 @@ __device__ __forceinline__ void lane_sums(double* buf, int lane, const double* v
     out[r][g] = s;
   }
   wave_sync();
+}
+template <int NR>
+__device__ __forceinline__ void lane_sums(double* buf, int lane, const double* v, double (*out)[GW]) {
+#pragma unroll
+  for (int r = 0; r < NR; ++r) buf[r * 64 + lane] = v[r];
+  lane_sums<NR>(buf, lane, out);
 }
 
 struct TermArgs {
@@ -122,31 +126,34 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
   double a[NS];
 #pragma unroll
   for (int m = 0; m < NS; ++m) a[m] = 0.0;
-  for (int t = 0; t < T.sh0[M]; ++t) {
-    const TermShell& q = T.sh[t];
-    const double dx = x - q.c[0], dy = y - q.c[1], dz = z - q.c[2];
-    const double r2 = dx * dx + dy * dy + dz * dz;
-    const double* C = mo + q.row * TERMS_LD;
+  for (int I = 0; I < M; ++I) {
+   const double dx = x - T.nuc[I][0], dy = y - T.nuc[I][1], dz = z - T.nuc[I][2];
+   const double r2 = dx * dx + dy * dy + dz * dz;
+   for (int t = T.sh0[I]; t < T.sh0[I + 1]; ++t) {
+    const TermShell q = T.sh[t];
+    const TermPrim* pr = T.pr + q.p0;
+    const double* C = mo + q.row * NS;
     by_count(q.np, [&](auto np) {
       constexpr int NP = decltype(np)::value;
       double s[3], p[3];
       if (q.sp) {
-        radial<NP, true, false>(q, r2, s, p);
+        radial<NP, true, false>(pr, r2, s, p);
         const double px = dx * p[0], py = dy * p[0], pz = dz * p[0];
 #pragma unroll
         for (int m = 0; m < NS; ++m) a[m] += C[m] * s[0];
 #pragma unroll
-        for (int m = 0; m < NS; ++m) a[m] += C[TERMS_LD + m] * px;
+        for (int m = 0; m < NS; ++m) a[m] += C[NS + m] * px;
 #pragma unroll
-        for (int m = 0; m < NS; ++m) a[m] += C[2 * TERMS_LD + m] * py;
+        for (int m = 0; m < NS; ++m) a[m] += C[2 * NS + m] * py;
 #pragma unroll
-        for (int m = 0; m < NS; ++m) a[m] += C[3 * TERMS_LD + m] * pz;
+        for (int m = 0; m < NS; ++m) a[m] += C[3 * NS + m] * pz;
       } else {
-        radial<NP, false, false>(q, r2, s, p);
+        radial<NP, false, false>(pr, r2, s, p);
 #pragma unroll
         for (int m = 0; m < NS; ++m) a[m] += C[m] * s[0];
       }
     });
+   }
   }
 
   // ---- inverse, one row per lane: Gauss-Jordan in place without row
@@ -218,31 +225,31 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
   // ---- determinant and electron-nucleus terms, nucleus by nucleus ----
   double gdx = 0.0, gdy = 0.0, gdz = 0.0, ld = 0.0;
   double gux = 0.0, guy = 0.0, guz = 0.0, lu = 0.0, u = 0.0, pot = 0.0;
-  double v6[18];
-  auto one_nucleus = [&](int I, double* o) {
+  auto one_nucleus = [&](int I, double* o) {  // o: the six rows of this nucleus at a stride of 64
     double ox = 0.0, oy = 0.0, oz = 0.0;
+    const double dx = x - T.nuc[I][0], dy = y - T.nuc[I][1], dz = z - T.nuc[I][2];
+    const double r2 = dx * dx + dy * dy + dz * dz;
     for (int t = T.sh0[I]; t < T.sh0[I + 1]; ++t) {
-      const TermShell& q = T.sh[t];
-      const double dx = x - q.c[0], dy = y - q.c[1], dz = z - q.c[2];
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      const double* C = mo + q.row * TERMS_LD;
+      const TermShell q = T.sh[t];
+      const TermPrim* pr = T.pr + q.p0;
+      const double* C = mo + q.row * NS;
       double ws = 0.0, wx = 0.0, wy = 0.0, wz = 0.0, s[3], p[3];
 #pragma unroll
       for (int m = 0; m < NS; ++m) ws += C[m] * col[m];
       if (q.sp) {
 #pragma unroll
-        for (int m = 0; m < NS; ++m) wx += C[TERMS_LD + m] * col[m];
+        for (int m = 0; m < NS; ++m) wx += C[NS + m] * col[m];
 #pragma unroll
-        for (int m = 0; m < NS; ++m) wy += C[2 * TERMS_LD + m] * col[m];
+        for (int m = 0; m < NS; ++m) wy += C[2 * NS + m] * col[m];
 #pragma unroll
-        for (int m = 0; m < NS; ++m) wz += C[3 * TERMS_LD + m] * col[m];
+        for (int m = 0; m < NS; ++m) wz += C[3 * NS + m] * col[m];
       }
       by_count(q.np, [&](auto np) {
         constexpr int NP = decltype(np)::value;
         if (q.sp)
-          radial<NP, true, true>(q, r2, s, p);
+          radial<NP, true, true>(pr, r2, s, p);
         else
-          radial<NP, false, true>(q, r2, s, p);
+          radial<NP, false, true>(pr, r2, s, p);
       });
       // s: grad = -2 R_a d, lap = -6 R_a + 4 r^2 R_aa; p_m = d_m R: grad_j =
       // delta_jm R - 2 d_m R_a d_j, lap = d_m (-10 R_a + 4 r^2 R_aa)
@@ -257,9 +264,8 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
       oy -= sy;
       oz -= sz;
     }
-    const double dx = x - S.nuc[I][0], dy = y - S.nuc[I][1], dz = z - S.nuc[I][2];
     double rr, ir;
-    qmc::M<double>::dist_inv(dx * dx + dy * dy + dz * dz, rr, ir);
+    qmc::M<double>::dist_inv(r2, rr, ir);
     pot -= S.Z[I] * ir;
     if (S.en_on) {
       double u1, lp;
@@ -278,11 +284,11 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
     if constexpr (DERIV) {
       for (int i = T.g0[sp][I]; i < T.g0[sp][I + 1]; ++i) {  // MO coefficients that follow R_I
         const TermMoGrp& G = T.grp[sp][i];
-        const TermShell& q = T.sh[G.sh];
-        const double ex = x - q.c[0], ey = y - q.c[1], ez = z - q.c[2];
+        const TermShell q = T.sh[G.sh];
+        const double ex = x - T.nuc[G.I][0], ey = y - T.nuc[G.I][1], ez = z - T.nuc[G.I][2];
         double s[3], p[3];
         by_count(q.np, [&](auto np) {
-          radial<decltype(np)::value, true, false>(q, ex * ex + ey * ey + ez * ez, s, p);
+          radial<decltype(np)::value, true, false>(T.pr + q.p0, ex * ex + ey * ey + ez * ez, s, p);
         });
         const double cv = L.cm[sp][G.mi][l];
         const double c0 = cv * s[0], c1 = cv * ex * p[0], c2 = cv * ey * p[0], c3 = cv * ez * p[0];
@@ -292,27 +298,27 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
       }
       const double f3 = rr > 1e-10 ? S.Z[I] * ir * ir * ir : 0.0;  // methane.rs:1253
       o[0] = ox;
-      o[1] = oy;
-      o[2] = oz;
-      o[3] = f3 * dx;
-      o[4] = f3 * dy;
-      o[5] = f3 * dz;
+      o[1 * 64] = oy;
+      o[2 * 64] = oz;
+      o[3 * 64] = f3 * dx;
+      o[4 * 64] = f3 * dy;
+      o[5 * 64] = f3 * dz;
     }
   };
   if constexpr (DERIV) {
+    double* o = row + lane;
     int I = 0;
     for (; I + 3 <= M; I += 3) {
-      one_nucleus(I, v6);
-      one_nucleus(I + 1, v6 + 6);
-      one_nucleus(I + 2, v6 + 12);
-      lane_sums<18>(row, lane, v6, &L.part[sp][6 * I]);
+#pragma unroll 1
+      for (int k = 0; k < 3; ++k) one_nucleus(I + k, o + 6 * 64 * k);
+      lane_sums<18>(row, lane, &L.part[sp][6 * I]);
     }
     for (; I < M; ++I) {
-      one_nucleus(I, v6);
-      lane_sums<6>(row, lane, v6, &L.part[sp][6 * I]);
+      one_nucleus(I, o);
+      lane_sums<6>(row, lane, &L.part[sp][6 * I]);
     }
   } else {
-    for (int I = 0; I < M; ++I) one_nucleus(I, v6);
+    for (int I = 0; I < M; ++I) one_nucleus(I, nullptr);
   }
 
   // ---- Jastrow partners and 1/r of the other electrons ----
@@ -333,7 +339,9 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
     pairsq += ok ? u1 * u1 : 0.0;
     pee += other ? ir : 0.0;
   };
+#pragma unroll 3
   for (int j = 0; j < NS; ++j) partner(sp * NS + j, true, j != slot);
+#pragma unroll 3
   for (int j = 0; j < NS; ++j) partner((1 - sp) * NS + j, false, true);
   const double gs = S.grad_scale;
   const double lj = (S.flags & F_J2_LAP_QUIRK) ? lu + pairsq : lu + gux * gux + guy * guy + guz * guz;
@@ -461,9 +469,10 @@ bool terms_table(const DevSys<double>& D, const MoDerivPair* pairs, const MoDeri
   if (D.jas_kind != JAS_PADE && D.jas_kind != JAS_NONE) return false;
   std::memset(&T, 0, sizeof T);
   T.n_nuc = D.n_nuc;
-  int rec_of[MAXSH], n = 0, row = 0;
+  int rec_of[MAXSH], n = 0, row = 0, prim = 0;
   for (int I = 0; I < D.n_nuc; ++I) {
     T.sh0[I] = n;
+    for (int c = 0; c < 3; ++c) T.nuc[I][c] = D.nuc[I][c];
     for (int i = 0; i < D.n_shell; ++i) {
       if (D.sh_center[i] != I) continue;
       const int kind = D.sh_kind[i], np = D.sh_nprim[i];
@@ -474,12 +483,12 @@ bool terms_table(const DevSys<double>& D, const MoDerivPair* pairs, const MoDeri
       q.sp = kind != SH_S;
       q.np = np == 1 ? 1 : np <= 3 ? 3 : 6;
       q.row = row;
-      for (int c = 0; c < 3; ++c) q.c[c] = D.nuc[I][c];
-      for (int k = 0; k < np; ++k) {
-        q.ex[k] = D.prim_exp[D.sh_prim0[i] + k];
-        q.cs[k] = kind == SH_P ? 0.0 : D.coef_s[D.sh_prim0[i] + k];
-        q.cp[k] = kind == SH_S ? 0.0 : D.coef_p[D.sh_prim0[i] + k];
-      }
+      q.p0 = prim;
+      if (prim + q.np > TERMS_PRIM) return false;
+      for (int k = 0; k < np; ++k)
+        T.pr[prim + k] = TermPrim{D.prim_exp[D.sh_prim0[i] + k], kind == SH_P ? 0.0 : D.coef_s[D.sh_prim0[i] + k],
+                                  kind == SH_S ? 0.0 : D.coef_p[D.sh_prim0[i] + k]};
+      prim += q.np;
       for (int r = kind == SH_P ? 1 : 0; r < rows; ++r)
         for (int s = 0; s < 2; ++s)
           for (int m = 0; m < NS; ++m) T.mo[s][row + r][m] = D.moT[s][D.sh_ao0[i] + r - (kind == SH_P ? 1 : 0)][m];
@@ -513,6 +522,7 @@ bool terms_table(const DevSys<double>& D, const MoDerivPair* pairs, const MoDeri
             ++ng;
             T.grp[s][g].sh = rec;
             T.grp[s][g].mi = mi;
+            T.grp[s][g].I = D.sh_center[sh];
           }
           T.grp[s][g].d[q][ents[k].c] += ents[k].d;
         }

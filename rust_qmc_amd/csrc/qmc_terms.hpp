@@ -15,22 +15,23 @@ constexpr int TERMS_W = 3;       // walkers per workgroup (63 of 64 lanes)
 constexpr int TERMS_MAXSH = 40;  // shells
 constexpr int TERMS_MAXP = 6;    // primitives per shell
 constexpr int TERMS_ROWS = 80;   // MO coefficient rows (AOs, and an s row for every p-only shell)
-constexpr int TERMS_LD = 24;     // doubles per row
+constexpr int TERMS_PRIM = 160;  // primitive slots
 constexpr int TERMS_MO = 6;      // distinct MOs whose coefficients follow the geometry
 constexpr int TERMS_GRP = 32;    // MO-derivative groups per spin
 
-// The system as the kernel reads it, all with wave-uniform addresses: the
-// shells sorted by centre, each record one block of scalar loads at a known
-// address (primitives zero-padded to 1, 3 or 6), the MO rows in the same
-// order so that they are walked with a running pointer.
+// The system as the kernel reads it, all with wave-uniform addresses and
+// packed, so that benzene's table (13.6 KB) stays in the 16 KB scalar cache:
+// the shells sorted by centre, their primitives zero-padded to 1, 3 or 6,
+// the MO rows in the same order.
 struct TermShell {
-  int sp, np, row, pad;  // 1: s and p parts (4 MO rows), 0: s only (1 row); padded primitive count; first MO row
-  double c[3];           // centre
-  double ex[TERMS_MAXP], cs[TERMS_MAXP], cp[TERMS_MAXP];
+  int sp, np, row, p0;  // 1: s and p parts (4 MO rows), 0: s only (1 row); padded primitive count; first row, slot
+};
+struct TermPrim {
+  double ex, cs, cp;
 };
 // d ln D / d R_{I,c} += sum_q d[q][c] (A^-1)_{m,k} chi_q(r_k), q the shell's s, px, py, pz
 struct TermMoGrp {
-  int sh, mi;  // shell record, index into mo_list
+  int sh, mi, I, pad;  // shell record, index into mo_list, the shell's centre
   double d[4][3];
 };
 struct TermTab {
@@ -38,8 +39,10 @@ struct TermTab {
   int sh0[MAXN + 1];       // shells of nucleus I: [sh0[I], sh0[I + 1])
   int g0[2][MAXN + 1];     // MO-derivative groups of (spin, nucleus)
   int mo_list[TERMS_MO];
+  double nuc[MAXN][3];
   TermShell sh[TERMS_MAXSH];
-  double mo[2][TERMS_ROWS][TERMS_LD];
+  TermPrim pr[TERMS_PRIM];
+  double mo[2][TERMS_ROWS][TERMS_N];
   TermMoGrp grp[2][TERMS_GRP];
 };
 
