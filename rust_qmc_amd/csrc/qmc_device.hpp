@@ -346,18 +346,30 @@ __device__ __forceinline__ void det_terms_w(const DevSys<T>& S, T x, T y, T z, W
         sl += wd * lr;
       }
     } else {
-      // radial STO: R' and R''; grad = R' d/s, lap = R'' + 2 R'/s
-      T s = M<T>::sq(r2);
+      // radial STO: R' and R''; grad = R' d/s, lap = R'' + 2 R'/s.  FP64
+      // takes s and 1/s from one reciprocal square root: the two IEEE
+      // divisions per primitive and the square root were half of its
+      // instructions.
+      T s, is;
+      if constexpr (sizeof(T) == 8)
+        M<T>::dist_inv(r2, s, is);
+      else
+        s = M<T>::sq(r2);
       T d1 = 0, d2 = 0;
       for (int k = 0; k < np; ++k) {
         const T zt = S.prim_exp[p0 + k];
         const int p = sh.pw(k);
         const T pf = T(p);
         // s^p, s^(p-1), s^(p-2) with the p = 0, 1 terms multiplied by zero
-        T sp = T(1);
+        T sp = T(1), spm1, spm2;
         for (int q = 0; q < p; ++q) sp *= s;
-        T spm1 = p >= 1 ? sp / s : T(0);
-        T spm2 = p >= 2 ? spm1 / s : T(0);
+        if constexpr (sizeof(T) == 8) {
+          spm1 = p >= 1 ? sp * is : T(0);
+          spm2 = p >= 2 ? spm1 * is : T(0);
+        } else {
+          spm1 = p >= 1 ? sp / s : T(0);
+          spm2 = p >= 2 ? spm1 / s : T(0);
+        }
         T e = S.coef_s[p0 + k] * prim_e(S, p0 + k, s);
         d1 += e * (-zt * sp + pf * spm1);
         d2 += e * (zt * zt * sp - T(2) * zt * pf * spm1 + pf * (pf - T(1)) * spm2);
@@ -366,7 +378,7 @@ __device__ __forceinline__ void det_terms_w(const DevSys<T>& S, T x, T y, T z, W
       if (s == T(0)) {
         sl = (kind == SH_SLATER1S) ? (w == T(0) ? T(0) : -INFINITY * w) : T(0);
       } else {
-        T is = T(1) / s;
+        if constexpr (sizeof(T) == 4) is = T(1) / s;
         T g = w * d1 * is;
         sx = g * dx;
         sy = g * dy;
