@@ -759,6 +759,118 @@ struct Staged {
   }
 };
 
+// The device side of one call: its host inputs, an int flag that starts at
+// zero, its host outputs and scratch, in that order (buffers the caller has
+// on the device are used where they are).  Up to 2 MiB is one allocation
+// instead of one per buffer, and up to 1 MiB each way is one copy: an
+// evaluation of 64 H2 configurations from host arrays took 133 us with seven
+// allocations and seven copies, 39 us with one and two.  Larger calls keep an
+// allocation per buffer (one block of 3 MiB cost more than seven small ones)
+// and copy straight to the caller.
+class CallBuffers {
+  static constexpr size_t kAlign = 256, kPack = 1 << 20, kOne = 2 << 20;
+  struct Buf {
+    const void* in;
+    void* out;
+    void* dev;
+    size_t bytes, off;
+    bool own;  // an allocation of its own
+  };
+  Buf b_[8];
+  int n_ = 0;
+  size_t need_ = 0, flag_off_ = 0, out_end_ = 0;
+  bool pack_in_ = false, pack_out_ = false;
+  char* base_ = nullptr;
+  hipStream_t st_;
+  std::vector<char> up_;  // the packed inputs, alive until the stream has drained
+  int add(const void* in, void* out, size_t bytes, bool dev) {
+    b_[n_] = Buf{in, out, dev ? const_cast<void*>(in ? in : out) : nullptr, bytes, 0, false};
+    if (!dev && (in || out || bytes)) {
+      b_[n_].off = need_;
+      need_ += (bytes + kAlign - 1) / kAlign * kAlign;
+    }
+    return n_++;
+  }
+
+ public:
+  explicit CallBuffers(hipStream_t st) : st_(st) {}
+  CallBuffers(const CallBuffers&) = delete;
+  ~CallBuffers() {
+    // hipFree waits for the device, also after an error return
+    if (base_) (void)hipFree(base_);
+    for (int i = 0; i < n_; ++i)
+      if (b_[i].own) (void)hipFree(b_[i].dev);
+  }
+  // inputs first, then flag(), then outputs, then scratch
+  int input(const void* p, size_t bytes) { return add(p, nullptr, bytes, is_device_ptr(p)); }
+  void flag() {
+    flag_off_ = need_;
+    need_ += kAlign;
+    out_end_ = flag_off_ + sizeof(int);
+  }
+  int output(void* p, size_t bytes) {
+    if (!p) return add(nullptr, nullptr, 0, true);
+    const int i = add(nullptr, p, bytes, is_device_ptr(p));
+    if (!b_[i].dev) out_end_ = b_[i].off + bytes;
+    return i;
+  }
+  int scratch(size_t bytes) { return add(nullptr, nullptr, bytes, false); }
+  template <class P>
+  P* get(int i) const {
+    return (P*)b_[i].dev;
+  }
+  int* flag_ptr() const { return (int*)(base_ + flag_off_); }
+
+  int open() {
+    const bool one = need_ <= kOne;
+    if (!one) flag_off_ = 0;
+    HIP_TRY(hipMalloc(&base_, one ? need_ : kAlign));
+    for (int i = 0; i < n_; ++i) {
+      if (b_[i].dev || !b_[i].bytes) continue;
+      if (one) {
+        b_[i].dev = base_ + b_[i].off;
+      } else {
+        HIP_TRY(hipMalloc(&b_[i].dev, b_[i].bytes));
+        b_[i].own = true;
+      }
+    }
+    pack_in_ = one && flag_off_ > 0 && flag_off_ + sizeof(int) <= kPack;
+    pack_out_ = one && out_end_ - flag_off_ <= kPack;
+    const size_t up = flag_off_ + sizeof(int);
+    if (pack_in_) {
+      up_.assign(up, 0);
+      for (int i = 0; i < n_; ++i)
+        if (b_[i].in && b_[i].dev != b_[i].in) std::memcpy(up_.data() + b_[i].off, b_[i].in, b_[i].bytes);
+      HIP_TRY(hipMemcpyAsync(base_, up_.data(), up, hipMemcpyHostToDevice, st_));
+      return QMC_OK;
+    }
+    for (int i = 0; i < n_; ++i)
+      if (b_[i].in && b_[i].dev != b_[i].in)
+        HIP_TRY(hipMemcpyAsync(b_[i].dev, b_[i].in, b_[i].bytes, hipMemcpyHostToDevice, st_));
+    HIP_TRY(hipMemsetAsync(flag_ptr(), 0, sizeof(int), st_));
+    return QMC_OK;
+  }
+  // outputs back, the stream drained; *flag receives the flag
+  int close(int* flag) {
+    if (pack_out_) {
+      const size_t back = out_end_ - flag_off_;
+      std::vector<char> h(back);
+      HIP_TRY(hipMemcpyAsync(h.data(), base_ + flag_off_, back, hipMemcpyDeviceToHost, st_));
+      HIP_TRY(hipStreamSynchronize(st_));
+      for (int i = 0; i < n_; ++i)
+        if (b_[i].out && b_[i].dev != b_[i].out) std::memcpy(b_[i].out, h.data() + (b_[i].off - flag_off_), b_[i].bytes);
+      std::memcpy(flag, h.data(), sizeof(int));
+      return QMC_OK;
+    }
+    for (int i = 0; i < n_; ++i)
+      if (b_[i].out && b_[i].dev != b_[i].out)
+        HIP_TRY(hipMemcpyAsync(b_[i].out, b_[i].dev, b_[i].bytes, hipMemcpyDeviceToHost, st_));
+    HIP_TRY(hipMemcpyAsync(flag, flag_ptr(), sizeof(int), hipMemcpyDeviceToHost, st_));
+    HIP_TRY(hipStreamSynchronize(st_));
+    return QMC_OK;
+  }
+};
+
 }  // namespace
 
 // ===========================================================================
@@ -1174,35 +1286,30 @@ int qmc_evaluate(const qmc_system* sys, int64_t W, const double* pos, double* lo
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   const int N = sys->h.n_elec();
-  Staged P, L, S, G, Lp, E;
-  if ((rc = P.init(pos, sizeof(double) * W * N * 3, true, st))) return rc;
-  if ((rc = L.init(logabs, sizeof(double) * W, false, st))) return rc;
-  if ((rc = S.init(sign, sizeof(double) * W, false, st))) return rc;
-  if ((rc = G.init(grad, sizeof(double) * W * N * 3, false, st))) return rc;
-  if ((rc = Lp.init(lap, sizeof(double) * W * N, false, st))) return rc;
-  if ((rc = E.init(eloc, sizeof(double) * W, false, st))) return rc;
-  int* sing = nullptr;
-  HIP_TRY(hipMalloc(&sing, sizeof(int)));
-  std::unique_ptr<int, void (*)(int*)> sing_guard(sing, [](int* p) { (void)hipFree(p); });
-  HIP_TRY(hipMemsetAsync(sing, 0, sizeof(int), st));
-  EvalOut O{(double*)L.dev, (double*)S.dev, (double*)G.dev, (double*)Lp.dev, (double*)E.dev};
+  CallBuffers B(st);
+  const int P = B.input(pos, sizeof(double) * W * N * 3);
+  B.flag();  // configurations with a singular Slater matrix
+  const int L = B.output(logabs, sizeof(double) * W), S = B.output(sign, sizeof(double) * W),
+            G = B.output(grad, sizeof(double) * W * N * 3), Lp = B.output(lap, sizeof(double) * W * N),
+            E = B.output(eloc, sizeof(double) * W);
+  if ((rc = B.open())) return rc;
+  int* sing = B.flag_ptr();
+  const double* p = B.get<double>(P);
+  EvalOut O{B.get<double>(L), B.get<double>(S), B.get<double>(G), B.get<double>(Lp), B.get<double>(E)};
   if (sys->use_terms()) {
-    HIP_TRY(terms_eval(sys->d64, sys->terms, W, (const double*)P.dev, O, sing, st));
+    HIP_TRY(terms_eval(sys->d64, sys->terms, W, p, O, sing, st));
   } else if (sys->wave()) {
     if (sys->precision == QMC_FP64)
-      HIP_TRY(wave_eval<double>(sys->d64, sys->d64, W, (const double*)P.dev, sys->shape(), O, sing, st));
+      HIP_TRY(wave_eval<double>(sys->d64, sys->d64, W, p, sys->shape(), O, sing, st));
     else
-      HIP_TRY(wave_eval<float>(sys->d64, sys->d32, W, (const double*)P.dev, sys->shape(), O, sing, st));
+      HIP_TRY(wave_eval<float>(sys->d64, sys->d32, W, p, sys->shape(), O, sing, st));
   } else if (sys->precision == QMC_FP64) {
-    HIP_TRY(sys->ops->eval64(sys->d64, sys->d64, W, (const double*)P.dev, O, sing, st));
+    HIP_TRY(sys->ops->eval64(sys->d64, sys->d64, W, p, O, sing, st));
   } else {
-    HIP_TRY(sys->ops->eval32(sys->d64, sys->d32, W, (const double*)P.dev, O, sing, st));
+    HIP_TRY(sys->ops->eval32(sys->d64, sys->d32, W, p, O, sing, st));
   }
-  for (Staged* s : {&L, &S, &G, &Lp, &E})
-    if ((rc = s->copy_out())) return rc;
   int nsing = 0;
-  HIP_TRY(hipMemcpyAsync(&nsing, sing, sizeof(int), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
+  if ((rc = B.close(&nsing))) return rc;
   if (nsing > 0 && !(sys->h.flags & QMC_FLAG_SINGULAR_IDENTITY))
     return fail(QMC_ERR_SINGULAR, std::to_string(nsing) + " configurations with a singular Slater matrix");
   return QMC_OK;
@@ -1221,6 +1328,8 @@ int qmc_local_energy(const qmc_system* s, int64_t W, const double* pos, double* 
   return qmc_evaluate(s, W, pos, nullptr, nullptr, nullptr, nullptr, el, st);
 }
 
+static_assert(3 * MAXN <= (int)(sizeof(DerivUnpack::fnn) / sizeof(double)), "fnn holds 3 MAXN forces");
+
 int qmc_derivatives(const qmc_system* sys, int64_t W, const double* pos, double* eloc, double* O, double* dE,
                     double* F, double* Om, void* stream) {
   if (!sys || !pos || W < 0) return fail(QMC_ERR_INVALID, "bad arguments");
@@ -1228,35 +1337,21 @@ int qmc_derivatives(const qmc_system* sys, int64_t W, const double* pos, double*
   hipStream_t st = (hipStream_t)stream;
   const int N = sys->h.n_elec();
   const Cols C(sys->h);
-  int rc;
-  Staged P;
-  if ((rc = P.init(pos, sizeof(double) * W * N * 3, true, st))) return rc;
-  double* Y = nullptr;
-  HIP_TRY(hipMalloc(&Y, sizeof(double) * (size_t)C.Qp * W));
-  std::unique_ptr<double, void (*)(double*)> yg(Y, [](double* p) { (void)hipFree(p); });
-  DerivArgs A{W, C.P, C.M, C.Qp, (const double*)P.dev, nullptr, nullptr, 0, Y, W};
+  int rc, flag = 0;
+  CallBuffers B(st);
+  const size_t w8 = sizeof(double) * W;
+  const int P = B.input(pos, w8 * N * 3);
+  B.flag();
+  const int iE = B.output(eloc, w8), iO = B.output(O, w8 * C.P), iD = B.output(dE, w8 * C.P),
+            iF = B.output(F, w8 * 3 * C.M), iM = B.output(Om, w8 * 3 * C.M), iY = B.scratch(w8 * C.Qp);
+  if ((rc = B.open())) return rc;
+  DerivArgs A{W, C.P, C.M, C.Qp, B.get<double>(P), nullptr, nullptr, 0, B.get<double>(iY), W};
   if ((rc = launch_derivs(sys, A, sys->precision, st))) return rc;
-  std::vector<double> h((size_t)C.Qp * W);
-  HIP_TRY(hipMemcpyAsync(h.data(), Y, h.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  const int Pn = C.P, M = C.M;
-  const std::vector<double> fnn = hf_nn(sys->h);
-  std::vector<double> o((size_t)W * Pn), d((size_t)W * Pn), f((size_t)W * 3 * M), om((size_t)W * 3 * M), e(W);
-  for (int64_t w = 0; w < W; ++w) {
-    e[w] = h[(size_t)C.e() * W + w];
-    for (int k = 0; k < Pn; ++k) {
-      o[w * Pn + k] = h[(size_t)k * W + w];
-      d[w * Pn + k] = h[(size_t)C.de(k) * W + w];
-    }
-    for (int q = 0; q < 3 * M; ++q) {
-      om[w * 3 * M + q] = h[(size_t)(Pn + q) * W + w];
-      f[w * 3 * M + q] = h[(size_t)C.f(q / 3, q % 3) * W + w] + fnn[q];
-    }
-  }
-  if ((rc = put(eloc, e.data(), e.size())) || (rc = put(O, o.data(), o.size())) || (rc = put(dE, d.data(), d.size())) ||
-      (rc = put(F, f.data(), f.size())) || (rc = put(Om, om.data(), om.size())))
-    return rc;
-  return QMC_OK;
+  DerivUnpack U{W, C.P, C.M, A.Y, B.get<double>(iE), B.get<double>(iO), B.get<double>(iD), B.get<double>(iF),
+                B.get<double>(iM), {}};
+  hf_nn_fill(sys->h, U.fnn);
+  HIP_TRY(launch_deriv_unpack(U, st));
+  return B.close(&flag);
 }
 
 int qmc_log_derivs(const qmc_system* s, int64_t W, const double* pos, double* O, void* st) {
@@ -1292,7 +1387,6 @@ int qmc_derivatives_noalloc(const qmc_system* sys, int64_t W, const double* pos,
   hipStream_t st = (hipStream_t)stream;
   DerivArgs A{W, C.P, C.M, C.Qp, pos, nullptr, nullptr, 0, Y, W};
   if (int rc = launch_derivs(sys, A, sys->precision, st)) return rc;
-  static_assert(3 * MAXN <= (int)(sizeof(DerivUnpack::fnn) / sizeof(double)), "fnn holds 3 MAXN forces");
   DerivUnpack U{W, C.P, C.M, Y, eloc, O, dE, F, Om, {}};
   hf_nn_fill(sys->h, U.fnn);
   HIP_TRY(launch_deriv_unpack(U, st));
