@@ -41,6 +41,7 @@ struct GroupShape {
   struct Lds {
     double mo[GroupAo<Bs>::v][2][NSP];  // MO coefficients [ao][spin][m], zero past the sector's size
     double xyz[WPB][N][3];
+    double prop[WPB][N][4];  // sweeps: each electron's proposal (or normals) and acceptance uniform
     double row[64][NS + 1];  // inverse rows in transit (odd stride: 64 lanes over all banks)
   };
 };
@@ -146,16 +147,23 @@ __device__ __forceinline__ PairSums group_pairs(const DevSys<double>& S, const L
 }
 
 // -1/2 lap psi / psi of one electron plus its potential share, from the
-// determinant terms of its weights and its pair sums (electron_terms)
+// determinant terms of its weights and its pair sums (electron_terms);
+// on_shell as det_terms_w, gd receives grad D / D
+template <class Bs, class Wgt, class OnShell>
+__device__ __forceinline__ double group_energy(const DevSys<double>& S, double x, double y, double z, Wgt wgt,
+                                               const PairSums& P, OnShell on_shell, double gd[3]) {
+  double ld;
+  det_terms_w<double, Wgt, OnShell, Bs>(S, x, y, z, wgt, gd[0], gd[1], gd[2], ld, on_shell);
+  const double gs = S.grad_scale;
+  const double lj = (S.flags & F_J2_LAP_QUIRK) ? P.lap + P.sq : P.lap + P.gx * P.gx + P.gy * P.gy + P.gz * P.gz;
+  const double lap = ld + lj + 2.0 * gs * (gd[0] * P.gx + gd[1] * P.gy + gd[2] * P.gz);
+  return -0.5 * lap + P.v;
+}
 template <class Bs, class Wgt>
 __device__ __forceinline__ double group_energy(const DevSys<double>& S, double x, double y, double z, Wgt wgt,
                                                const PairSums& P) {
-  double gdx, gdy, gdz, ld;
-  det_terms_w<double, Wgt, NoShell, Bs>(S, x, y, z, wgt, gdx, gdy, gdz, ld, NoShell{});
-  const double gs = S.grad_scale;
-  const double lj = (S.flags & F_J2_LAP_QUIRK) ? P.lap + P.sq : P.lap + P.gx * P.gx + P.gy * P.gy + P.gz * P.gz;
-  const double lap = ld + lj + 2.0 * gs * (gdx * P.gx + gdy * P.gy + gdz * P.gz);
-  return -0.5 * lap + P.v;
+  double gd[3];
+  return group_energy<Bs>(S, x, y, z, wgt, P, NoShell{}, gd);
 }
 
 // Both sectors' Slater matrices inverted at once, one row (electron) per

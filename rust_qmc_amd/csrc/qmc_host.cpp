@@ -563,6 +563,18 @@ int need_engine(const qmc_system* s) {
   return QMC_OK;
 }
 
+// The lane-group engine takes work of few walkers for a compiled shell
+// structure without Pade series terms, in FP64 (its derivatives and
+// evaluations also for mixed precision); max_w is the kernel's GroupOps limit.
+bool group_fits(const qmc_system* s, int64_t W, int64_t GroupOps::*max_w) {
+  return s->engine == QMC_ENGINE_AUTO && !s->wave() && s->no_series() && s->h.mo_rule == QMC_MO_FIXED && s->gops &&
+         s->gops->derivs_ns && W <= s->gops->*max_w;
+}
+bool group_sweeps(const qmc_system* s, int prec, int64_t W) {
+  return prec == QMC_FP64 && group_fits(s, W, &GroupOps::w_sweep);
+}
+int64_t group_blocks(const qmc_system* s, int64_t W) { return (W + s->gops->wpb - 1) / s->gops->wpb; }
+
 // The derivative matrix Y of A.W walkers in the arithmetic type prec (FP64
 // in the one-electron-per-lane kernel, which serves both precisions): that
 // kernel for the 21 + 21-electron systems it fits, else the wave derivative
@@ -571,6 +583,10 @@ int need_engine(const qmc_system* s) {
 int launch_derivs(const qmc_system* s, DerivArgs A, int32_t prec, hipStream_t st) {
   if (s->use_terms()) {
     HIP_TRY(terms_derivs(s->d64, s->terms, A, st));
+    return QMC_OK;
+  }
+  if (group_fits(s, A.W, &GroupOps::w_deriv)) {
+    HIP_TRY(s->gops->derivs_ns(s->d64, A, st));
     return QMC_OK;
   }
   if (s->wave() || !s->dops || s->h.mo_rule != QMC_MO_FIXED) {
@@ -1298,6 +1314,8 @@ int qmc_evaluate(const qmc_system* sys, int64_t W, const double* pos, double* lo
   EvalOut O{B.get<double>(L), B.get<double>(S), B.get<double>(G), B.get<double>(Lp), B.get<double>(E)};
   if (sys->use_terms()) {
     HIP_TRY(terms_eval(sys->d64, sys->terms, W, p, O, sing, st));
+  } else if (group_fits(sys, W, &GroupOps::w_eval)) {
+    HIP_TRY(sys->gops->eval_ns(sys->d64, W, p, O, sing, st));
   } else if (sys->wave()) {
     if (sys->precision == QMC_FP64)
       HIP_TRY(wave_eval<double>(sys->d64, sys->d64, W, p, sys->shape(), O, sing, st));
@@ -1342,16 +1360,43 @@ int qmc_derivatives(const qmc_system* sys, int64_t W, const double* pos, double*
   const size_t w8 = sizeof(double) * W;
   const int P = B.input(pos, w8 * N * 3);
   B.flag();
-  const int iE = B.output(eloc, w8), iO = B.output(O, w8 * C.P), iD = B.output(dE, w8 * C.P),
-            iF = B.output(F, w8 * 3 * C.M), iM = B.output(Om, w8 * 3 * C.M), iY = B.scratch(w8 * C.Qp);
+  // a feature matrix of up to 128 KiB comes back whole and is taken apart on
+  // the host, which costs less than a kernel of its own (64 H2 configurations
+  // 44 us against 48); larger ones are unpacked on the device
+  std::vector<double> h;
+  if (w8 * C.Qp <= 131072) h.resize((size_t)W * C.Qp);
+  const auto dev = [&](double* p) { return h.empty() ? p : nullptr; };
+  const int iE = B.output(dev(eloc), w8), iO = B.output(dev(O), w8 * C.P), iD = B.output(dev(dE), w8 * C.P),
+            iF = B.output(dev(F), w8 * 3 * C.M), iM = B.output(dev(Om), w8 * 3 * C.M),
+            iY = h.empty() ? B.scratch(w8 * C.Qp) : B.output(h.data(), w8 * C.Qp);
   if ((rc = B.open())) return rc;
   DerivArgs A{W, C.P, C.M, C.Qp, B.get<double>(P), nullptr, nullptr, 0, B.get<double>(iY), W};
   if ((rc = launch_derivs(sys, A, sys->precision, st))) return rc;
-  DerivUnpack U{W, C.P, C.M, A.Y, B.get<double>(iE), B.get<double>(iO), B.get<double>(iD), B.get<double>(iF),
-                B.get<double>(iM), {}};
-  hf_nn_fill(sys->h, U.fnn);
-  HIP_TRY(launch_deriv_unpack(U, st));
-  return B.close(&flag);
+  if (h.empty()) {
+    DerivUnpack U{W, C.P, C.M, A.Y, B.get<double>(iE), B.get<double>(iO), B.get<double>(iD), B.get<double>(iF),
+                  B.get<double>(iM), {}};
+    hf_nn_fill(sys->h, U.fnn);
+    HIP_TRY(launch_deriv_unpack(U, st));
+    return B.close(&flag);
+  }
+  if ((rc = B.close(&flag))) return rc;
+  const int Pn = C.P, M3 = 3 * C.M;
+  const std::vector<double> fnn = hf_nn(sys->h);
+  std::vector<double> o((size_t)W * Pn), d((size_t)W * Pn), f((size_t)W * M3), om((size_t)W * M3);
+  for (int64_t w = 0; w < W; ++w) {
+    for (int k = 0; k < Pn; ++k) {
+      o[w * Pn + k] = h[(size_t)k * W + w];
+      d[w * Pn + k] = h[(size_t)C.de(k) * W + w];
+    }
+    for (int q = 0; q < M3; ++q) {
+      om[w * M3 + q] = h[(size_t)(Pn + q) * W + w];
+      f[w * M3 + q] = h[(size_t)C.f(q / 3, q % 3) * W + w] + fnn[q];
+    }
+  }
+  if ((rc = put(eloc, h.data() + (size_t)C.e() * W, W)) || (rc = put(O, o.data(), o.size())) ||
+      (rc = put(dE, d.data(), d.size())) || (rc = put(F, f.data(), f.size())) || (rc = put(Om, om.data(), om.size())))
+    return rc;
+  return QMC_OK;
 }
 
 int qmc_log_derivs(const qmc_system* s, int64_t W, const double* pos, double* O, void* st) {
@@ -1515,6 +1560,7 @@ int64_t sweep_blocks(const qmc_ensemble* e) {
   const qmc_system* s = e->sys;
   if (s->tile_sweeps(e->prec)) return tile_blocks(e->W);
   if (s->wave()) return e->W;
+  if (group_sweeps(s, e->prec, e->W)) return group_blocks(s, e->W);
   return (e->W + 63) / 64;
 }
 
@@ -1532,6 +1578,8 @@ int enqueue_single_sweeps(qmc_ensemble* e, const SweepArgs& A, double* trace, hi
       HIP_TRY(wave_sweep<double>(s->d64, e->view<double>(), s->shape(), A, e->partial, trace, st));
     else
       HIP_TRY(wave_sweep<float>(s->d32, e->view<float>(), s->shape(), A, e->partial, trace, st));
+  } else if (group_sweeps(s, e->prec, e->W)) {
+    HIP_TRY(s->gops->sweep64_ns(s->d64, e->view<double>(), A, e->partial, trace, st));
   } else {
     const bool no_series = s->h.k_ee == 0 && s->h.k_en == 0;
     if (e->prec == QMC_FP64)
@@ -1661,8 +1709,9 @@ int qmc_ensemble_sweeps(qmc_ensemble* e, const qmc_sweep_params* p, double* e_su
   const int nblk = p->move == QMC_MOVE_SINGLE ? (int)sweep_blocks(e)
                    : tdd                       ? (int)tile_blocks(e->W)
                    : wave                      ? (int)e->W
-                   : p->move == QMC_MOVE_ALL   ? (int)((e->W + s->gops->wpb - 1) / s->gops->wpb)
-                                               : (int)((e->W + 63) / 64);
+                   : p->move == QMC_MOVE_ALL || group_sweeps(s, e->prec, e->W)
+                       ? (int)group_blocks(s, e->W)
+                       : (int)((e->W + 63) / 64);
   const int refresh = p->refresh_interval > 0 ? p->refresh_interval : 0;
   int chunk = p->steps_per_launch > 0 ? p->steps_per_launch : 16;
   if ((rc = ensure_cap(&e->partial, &e->partial_cap, (size_t)chunk * nblk * 3))) return rc;
@@ -1699,6 +1748,8 @@ int qmc_ensemble_sweeps(qmc_ensemble* e, const qmc_sweep_params* p, double* e_su
         HIP_TRY(wave_dd<double>(s->d64, e->view<double>(), s->shape(), A, e->partial, trace, e->st));
       else if (wave)
         HIP_TRY(wave_dd<float>(s->d32, e->view<float>(), s->shape(), A, e->partial, trace, e->st));
+      else if (group_sweeps(s, e->prec, e->W))
+        HIP_TRY(s->gops->dd64_ns(s->d64, e->view<double>(), A, e->partial, trace, e->st));
       else if (e->prec == QMC_FP64)
         HIP_TRY((s->no_series() ? s->ops->dd64_ns : s->ops->dd64)(s->d64, e->view<double>(), A, e->partial, trace,
                                                                     e->st));
@@ -2634,10 +2685,15 @@ int isdmc_steps(const qmc_system* s, const qmc_isdmc_params* p, uint64_t seed, i
   const int N = s->h.n_elec(), M = s->h.n_nuc(), nu = s->h.n_up(), nd = s->h.n_dn();
   const int nainv = nu * nu + nd * nd;
   const int64_t T_all = p->n_burnin + p->n_steps;
-  // sweep partial rows: one per 64 walkers (register engine) or per walker (wave engine)
+  // sweep partial rows: one per 64 walkers (register engine), per block of
+  // the lane-group engine or per walker (wave engine)
   const bool wave = s->wave();
-  const int nb = (int)(cap / DMC_BLOCK), sweep_bs = wave ? 1 : 64, sweep_rows = (int)(cap / sweep_bs);
   const bool f64 = sizeof(T) == 8;
+  // one-step launches: the lane groups' longer prologue pays for 16 lanes a
+  // walker (CH4) only; H2 took 27.9 us per step with them, 27.7 without
+  const bool group = f64 && group_sweeps(s, QMC_FP64, p->n_walkers) && s->gops->wpb <= 4;
+  const int nb = (int)(cap / DMC_BLOCK), sweep_bs = wave ? 1 : (group ? s->gops->wpb : 64),
+            sweep_rows = (int)(cap / sweep_bs);
   // a stream of its own (graphs cannot capture the null stream) and the
   // two-step graphs, one per parity of the buffer a pair of steps starts in
   hipStream_t st = nullptr;
@@ -2721,6 +2777,8 @@ int isdmc_steps(const qmc_system* s, const qmc_isdmc_params* p, uint64_t seed, i
     if constexpr (sizeof(T) == 8) {
       if (wave)
         HIP_TRY(wave_dd<double>(s->d64, V[c], s->shape(), sa, partial, nullptr, st));
+      else if (group)
+        HIP_TRY(s->gops->dd64_ns(s->d64, V[c], sa, partial, nullptr, st));
       else
         HIP_TRY((s->no_series() ? s->ops->dd64_ns : s->ops->dd64)(s->d64, V[c], sa, partial, nullptr, st));
     } else {

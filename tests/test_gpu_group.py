@@ -73,3 +73,83 @@ def test_all_electron_mixed_follows_the_wave_engine(Q):
     assert np.array_equal(a[1], b[1])
     np.testing.assert_array_equal(a[3], b[3])
     np.testing.assert_allclose(a[2], b[2], rtol=2e-4, atol=1e-3)
+
+
+@pytest.mark.parametrize("move", ["single", "drift"])
+@pytest.mark.parametrize("W", [1, 5, 67, 130])
+@pytest.mark.parametrize("name", ["h2", "li", "li-ref", "ch4-sto3g", "ch4-631g"])
+def test_fp64_sweeps_match_register_engine(Q, name, W, move):
+    """Metropolis and drift-diffusion sweeps of every compiled structure
+    against the one-walker-per-lane kernels: the same decisions, positions
+    and energies to FP64 rounding (1e-9, as above)."""
+    s = {"h2": lambda: Q.H2MoleculeMO(), "li": lambda: Q.Lithium(0), "li-ref": lambda: Q.Lithium(),
+         "ch4-sto3g": lambda: Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0), "ch4-631g": lambda: Q.MethaneGTO()}[name]()
+    kw = dict(move=Q.QMC_MOVE_SINGLE if move == "single" else Q.QMC_MOVE_DRIFT, steps_per_launch=3, refresh_interval=5,
+              max_drift=0.5)
+    step = 0.3 if move == "single" else 0.02
+    a = _chain(Q, s, "auto", W, 8, step, **kw)
+    b = _chain(Q, s, "register", W, 8, step, **kw)
+    assert np.array_equal(a[1], b[1]) and b[1].sum() > 0
+    np.testing.assert_allclose(a[3], b[3], rtol=0, atol=1e-9)
+    for x, y in zip((a[0], a[2], *a[4]), (b[0], b[2], *b[4])):
+        np.testing.assert_allclose(x, y, rtol=1e-9, atol=1e-9)
+
+
+def test_fp64_sweeps_of_an_en_jastrow_on_h2(Q):
+    """H2's two lanes hold the electrons, so its nuclei take a second partner
+    round: a Pade Jastrow on the H2 shell structure."""
+    s = Q.System.from_desc(dict(
+        spins=[1, -1], nuclei=[[0, 0, 0.7], [0, 0, -0.7]], charges=[1.0, 1.0], aos=[(2, 0, 0, 0, 1, 0), (2, 1, 0, 0, 1, 1)],
+        prim_exp=[1.3, 1.3], prim_coef=[1.0, 1.0], prim_pow=[0, 0], mo_up=[[1.0, 1.0]], jastrow_kind=2, b_ee=1.1, b_en=1.6,
+        init_nuc=[0, 1]))
+    assert s.engine_name() == "register/h2-slater1s"
+    for move in (Q.QMC_MOVE_SINGLE, Q.QMC_MOVE_DRIFT):
+        a = _chain(Q, s, "auto", 67, 6, 0.05, move=move)
+        b = _chain(Q, s, "register", 67, 6, 0.05, move=move)
+        assert np.array_equal(a[1], b[1])
+        np.testing.assert_allclose(a[2], b[2], rtol=1e-9, atol=1e-9)
+        np.testing.assert_allclose(a[3], b[3], rtol=0, atol=1e-9)
+
+
+@pytest.mark.parametrize("W", [1, 3, 67])
+@pytest.mark.parametrize("name", ["h2", "li", "li-ref", "ch4-sto3g", "ch4-631g"])
+def test_derivatives_match_register_engine(Q, name, W):
+    """E_L, O, dE_L/dp, F and Omega of every compiled structure against the
+    one-walker-per-lane kernels, 1e-9 of each output's scale."""
+    s = {"h2": lambda: Q.H2MoleculeMO(), "li": lambda: Q.Lithium(0), "li-ref": lambda: Q.Lithium(),
+         "ch4-sto3g": lambda: Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0), "ch4-631g": lambda: Q.MethaneGTO()}[name]()
+    pos = 0.8 * np.random.default_rng(W).normal(size=(W, s.n_elec, 3))
+    s.set_engine("auto")
+    a = s.derivatives_batch(pos)
+    s.set_engine("register")
+    b = s.derivatives_batch(pos)
+    for k in b:
+        if b[k].size:
+            assert np.abs(a[k] - b[k]).max() <= 1e-9 * max(1.0, np.abs(b[k]).max()), k
+
+
+@pytest.mark.parametrize("W", [1, 3, 67])
+@pytest.mark.parametrize("name", ["h2", "li", "li-ref", "ch4-sto3g", "ch4-631g"])
+def test_evaluation_matches_register_engine(Q, name, W):
+    """ln|psi|, sign, gradients, Laplacians and E_L, 1e-9 of each output's scale."""
+    s = {"h2": lambda: Q.H2MoleculeMO(), "li": lambda: Q.Lithium(0), "li-ref": lambda: Q.Lithium(),
+         "ch4-sto3g": lambda: Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0), "ch4-631g": lambda: Q.MethaneGTO()}[name]()
+    pos = 0.8 * np.random.default_rng(W).normal(size=(W, s.n_elec, 3))
+    s.set_engine("auto")
+    a = s.evaluate_batch(pos)
+    s.set_engine("register")
+    b = s.evaluate_batch(pos)
+    for k in b:
+        assert np.abs(a[k] - b[k]).max() <= 1e-9 * max(1.0, np.abs(b[k]).max()), k
+
+
+def test_singular_configuration_is_reported(Q):
+    s = Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0)
+    pos = 0.8 * np.random.default_rng(5).normal(size=(6, 10, 3))
+    pos[4, 0] = 1e4  # every orbital of this electron underflows to zero
+    s.set_flags(0)
+    with pytest.raises(Q.QmcError, match="1 configurations with a singular"):
+        s.evaluate_batch(pos)
+    s.set_flags(Q.QMC_FLAGS_REFERENCE)
+    o = s.evaluate_batch(pos)
+    assert o["logabs"][4] == -np.inf and o["sign"][4] == 0.0 and np.isfinite(o["logabs"][:4]).all()
