@@ -12,6 +12,7 @@
 #include <cstring>
 
 #include "qmc_pair_terms.hpp"
+#include "qmc_terms_dev.hpp"
 #include "qmc_wave_dev.hpp"
 
 namespace qmc {
@@ -30,43 +31,6 @@ struct TermLds {
   double part[2][6 * MAXN][GW];    // per wavefront: Omega and F sums of its electrons
   double sums[2][9][GW];
 };
-
-// radial sums of a shell: R = sum c e, and with DER R_a = sum c a e and
-// R_aa = sum c a^2 e
-template <int NP, bool P, bool DER>
-__device__ __forceinline__ void radial(const TermPrim* q, double r2, double s[3], double p[3]) {
-#pragma unroll
-  for (int k = 0; k < 3; ++k) s[k] = p[k] = 0.0;
-#pragma unroll
-  for (int k = 0; k < NP; ++k) {
-    const double a = q[k].ex, e = M<double>::exn(-a * r2);
-    const double cs = q[k].cs * e;
-    s[0] += cs;
-    if constexpr (DER) {
-      s[1] += cs * a;
-      s[2] += cs * a * a;
-    }
-    if constexpr (P) {
-      const double cp = q[k].cp * e;
-      p[0] += cp;
-      if constexpr (DER) {
-        p[1] += cp * a;
-        p[2] += cp * a * a;
-      }
-    }
-  }
-}
-
-// f(integral_constant NP) for the shell's padded primitive count
-template <class F>
-__device__ __forceinline__ void by_count(int np, F f) {
-  if (np == 1)
-    f(std::integral_constant<int, 1>{});
-  else if (np == 3)
-    f(std::integral_constant<int, 3>{});
-  else
-    f(std::integral_constant<int, 6>{});
-}
 
 // sums over the 21 electrons of each walker of the NR (at most 20) values
 // per lane that this wavefront stored at buf[r * 64 + lane]: out[r][g]
@@ -127,33 +91,26 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
 #pragma unroll
   for (int m = 0; m < NS; ++m) a[m] = 0.0;
   for (int I = 0; I < M; ++I) {
-   const double dx = x - T.nuc[I][0], dy = y - T.nuc[I][1], dz = z - T.nuc[I][2];
-   const double r2 = dx * dx + dy * dy + dz * dz;
-   for (int t = T.sh0[I]; t < T.sh0[I + 1]; ++t) {
-    const TermShell q = T.sh[t];
-    const TermPrim* pr = T.pr + q.p0;
-    const double* C = mo + q.row * NS;
-    by_count(q.np, [&](auto np) {
+    const double dx = x - T.nuc[I][0], dy = y - T.nuc[I][1], dz = z - T.nuc[I][2];
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    nucleus_shells(T, I, [&](auto np, auto is_sp, const TermPrim* pr, int row) {
       constexpr int NP = decltype(np)::value;
+      constexpr bool SP = decltype(is_sp)::value;
+      const double* C = mo + row * NS;
       double s[3], p[3];
-      if (q.sp) {
-        radial<NP, true, false>(pr, r2, s, p);
-        const double px = dx * p[0], py = dy * p[0], pz = dz * p[0];
+      radial<NP, SP, false>(pr, r2, s, p);
 #pragma unroll
-        for (int m = 0; m < NS; ++m) a[m] += C[m] * s[0];
+      for (int m = 0; m < NS; ++m) a[m] += C[m] * s[0];
+      if constexpr (SP) {
+        const double px = dx * p[0], py = dy * p[0], pz = dz * p[0];
 #pragma unroll
         for (int m = 0; m < NS; ++m) a[m] += C[NS + m] * px;
 #pragma unroll
         for (int m = 0; m < NS; ++m) a[m] += C[2 * NS + m] * py;
 #pragma unroll
         for (int m = 0; m < NS; ++m) a[m] += C[3 * NS + m] * pz;
-      } else {
-        radial<NP, false, false>(pr, r2, s, p);
-#pragma unroll
-        for (int m = 0; m < NS; ++m) a[m] += C[m] * s[0];
       }
     });
-   }
   }
 
   // ---- inverse, one row per lane: Gauss-Jordan in place without row
@@ -229,14 +186,15 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
     double ox = 0.0, oy = 0.0, oz = 0.0;
     const double dx = x - T.nuc[I][0], dy = y - T.nuc[I][1], dz = z - T.nuc[I][2];
     const double r2 = dx * dx + dy * dy + dz * dz;
-    for (int t = T.sh0[I]; t < T.sh0[I + 1]; ++t) {
-      const TermShell q = T.sh[t];
-      const TermPrim* pr = T.pr + q.p0;
-      const double* C = mo + q.row * NS;
+    nucleus_shells(T, I, [&](auto np, auto is_sp, const TermPrim* pr, int row) {
+      constexpr int NP = decltype(np)::value;
+      constexpr bool SP = decltype(is_sp)::value;
+      const double* C = mo + row * NS;
       double ws = 0.0, wx = 0.0, wy = 0.0, wz = 0.0, s[3], p[3];
+      radial<NP, SP, true>(pr, r2, s, p);
 #pragma unroll
       for (int m = 0; m < NS; ++m) ws += C[m] * col[m];
-      if (q.sp) {
+      if constexpr (SP) {
 #pragma unroll
         for (int m = 0; m < NS; ++m) wx += C[NS + m] * col[m];
 #pragma unroll
@@ -244,13 +202,6 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
 #pragma unroll
         for (int m = 0; m < NS; ++m) wz += C[3 * NS + m] * col[m];
       }
-      by_count(q.np, [&](auto np) {
-        constexpr int NP = decltype(np)::value;
-        if (q.sp)
-          radial<NP, true, true>(pr, r2, s, p);
-        else
-          radial<NP, false, true>(pr, r2, s, p);
-      });
       // s: grad = -2 R_a d, lap = -6 R_a + 4 r^2 R_aa; p_m = d_m R: grad_j =
       // delta_jm R - 2 d_m R_a d_j, lap = d_m (-10 R_a + 4 r^2 R_aa)
       const double wd = wx * dx + wy * dy + wz * dz;
@@ -263,7 +214,7 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
       ox -= sx;
       oy -= sy;
       oz -= sz;
-    }
+    });
     double rr, ir;
     qmc::M<double>::dist_inv(r2, rr, ir);
     pot -= S.Z[I] * ir;
@@ -498,6 +449,14 @@ bool terms_table(const DevSys<double>& D, const MoDerivPair* pairs, const MoDeri
   }
   T.sh0[D.n_nuc] = n;
   if (n != D.n_shell) return false;
+  for (int I = 0; I < D.n_nuc; ++I) {
+    const TermShell* q = T.sh + T.sh0[I];
+    const int k = T.sh0[I + 1] - T.sh0[I];
+    auto is = [&](int i, int np, int sp) { return q[i].np == np && q[i].sp == sp; };
+    T.pat[I] = k == 3 && is(0, 6, 0) && is(1, 3, 1) && is(2, 1, 1) ? TERMS_PAT_631G
+               : k == 2 && is(0, 3, 0) && is(1, 1, 0)             ? TERMS_PAT_631G_H
+                                                                  : TERMS_PAT_ANY;
+  }
   T.same = std::memcmp(T.mo[0], T.mo[1], sizeof T.mo[0]) == 0;
   // MO-derivative groups: (spin, nucleus, shell, MO) with its 4 x 3 matrix
   for (int s = 0; s < 2; ++s) {

@@ -19,6 +19,12 @@ constexpr int TERMS_PRIM = 160;  // primitive slots
 constexpr int TERMS_MO = 6;      // distinct MOs whose coefficients follow the geometry
 constexpr int TERMS_GRP = 32;    // MO-derivative groups per spin
 
+// Shell patterns of a nucleus that are compiled: the 6-31G ones of a
+// first-row atom (s of 6 primitives, sp of 3, sp of 1) and of hydrogen (s of
+// 3, s of 1), whose shells then form one block of straight-line code; any
+// other nucleus runs shell by shell.
+enum : int { TERMS_PAT_ANY = 0, TERMS_PAT_631G = 1, TERMS_PAT_631G_H = 2 };
+
 // The system as the kernel reads it, all with wave-uniform addresses and
 // packed, so that benzene's table (13.6 KB) stays in the 16 KB scalar cache:
 // the shells sorted by centre, their primitives zero-padded to 1, 3 or 6,
@@ -37,6 +43,7 @@ struct TermMoGrp {
 struct TermTab {
   int n_nuc, n_mo, same;   // same: both spins' MO rows are equal
   int sh0[MAXN + 1];       // shells of nucleus I: [sh0[I], sh0[I + 1])
+  int pat[MAXN];           // their pattern (TERMS_PAT_*)
   int g0[2][MAXN + 1];     // MO-derivative groups of (spin, nucleus)
   int mo_list[TERMS_MO];
   double nuc[MAXN][3];
