@@ -195,9 +195,11 @@ int qmc_set_precision(qmc_system* sys, int32_t precision);
 #define QMC_ENGINE_GENERIC 3
 #define QMC_ENGINE_TILE 4
 int qmc_set_engine(qmc_system* sys, int32_t engine);
-/* Name of the kernels a system's sweeps run on: "tile", "wave",
+/* Name of the engine a system's sweeps run on: "tile", "wave",
  * "register/generic" or "register/<shell structure>" (no reference
- * counterpart; diagnostics). */
+ * counterpart; diagnostics).  Under AUTO, FP64 sweeps of a "tile" system and
+ * FP64 sweeps of few walkers of a "register" one run on that engine's
+ * kernels with more lanes per walker (32, and one per electron). */
 int qmc_engine_name(const qmc_system* sys, char* buf, int32_t len);
 int qmc_set_flags(qmc_system* sys, uint32_t flags);
 int qmc_system_info(const qmc_system* sys, int32_t* n_elec, int32_t* n_up, int32_t* n_nuc, int32_t* n_ao);

@@ -20,6 +20,7 @@
 #include "qmc_device.hpp"
 #include "qmc_dmc.hpp"
 #include "qmc_group.hpp"
+#include "qmc_half.hpp"
 #include "qmc_kernels.hpp"
 #include "qmc_noalloc.hpp"
 #include "qmc_refresh.hpp"
@@ -158,6 +159,10 @@ struct qmc_system {
   bool terms_ok = false;
   // evaluation and derivatives one electron per lane, unless the wave engine is selected
   bool use_terms() const { return wave() && terms_ok && engine != QMC_ENGINE_WAVE; }
+  bool half_ok = false;
+  // FP64 sweeps on the half-wave engine; the tile engine keeps mixed
+  // precision and the Jastrows with series terms
+  bool use_half(int32_t prec) const { return prec == QMC_FP64 && wave() && half_ok && engine == QMC_ENGINE_AUTO; }
   ~qmc_system() {
     if (terms) (void)hipFree(terms);
     if (d64) (void)hipFree(d64);
@@ -459,6 +464,7 @@ int upload(qmc_system* s) {
     }
     auto tab = std::make_unique<TermTab>();
     s->terms_ok = terms_table(*d64, pairs.data(), ents.data(), s->mdp0, *tab);
+    s->half_ok = s->terms_ok && half_fits(*tab);
     if (s->terms_ok) {
       if (!s->terms) HIP_TRY(hipMalloc(&s->terms, sizeof(TermTab)));
       HIP_TRY(hipMemcpy(s->terms, tab.get(), sizeof(TermTab), hipMemcpyHostToDevice));
@@ -1558,6 +1564,7 @@ int ensure_cap(double** p, size_t* cap, size_t n) {
 // blocks (partial-sum rows) of one single-electron sweep launch of e
 int64_t sweep_blocks(const qmc_ensemble* e) {
   const qmc_system* s = e->sys;
+  if (s->use_half(e->prec)) return half_blocks(e->W);
   if (s->tile_sweeps(e->prec)) return tile_blocks(e->W);
   if (s->wave()) return e->W;
   if (group_sweeps(s, e->prec, e->W)) return group_blocks(s, e->W);
@@ -1568,7 +1575,9 @@ int64_t sweep_blocks(const qmc_ensemble* e) {
 // system selects (partial sums into e->partial)
 int enqueue_single_sweeps(qmc_ensemble* e, const SweepArgs& A, double* trace, hipStream_t st) {
   const qmc_system* s = e->sys;
-  if (s->tile_sweeps(e->prec)) {
+  if (s->use_half(e->prec)) {
+    HIP_TRY(half_sweep(s->d64, s->terms, e->view<double>(), A, e->partial, trace, st));
+  } else if (s->tile_sweeps(e->prec)) {
     if (e->prec == QMC_FP64)
       HIP_TRY(tile_sweep<double>(s->d64, e->view<double>(), s->tile, A, e->partial, trace, st));
     else
@@ -1705,8 +1714,10 @@ int qmc_ensemble_sweeps(qmc_ensemble* e, const qmc_sweep_params* p, double* e_su
   // drift-diffusion moves on the tile engine where it runs single-electron
   // sweeps; all-electron moves on the wave engine (also for tile-engine
   // systems): one block per walker
-  const bool tdd = p->move == QMC_MOVE_DRIFT && s->tile_dd(e->prec);
+  const bool hdd = p->move == QMC_MOVE_DRIFT && s->use_half(e->prec);
+  const bool tdd = p->move == QMC_MOVE_DRIFT && !hdd && s->tile_dd(e->prec);
   const int nblk = p->move == QMC_MOVE_SINGLE ? (int)sweep_blocks(e)
+                   : hdd                       ? (int)half_blocks(e->W)
                    : tdd                       ? (int)tile_blocks(e->W)
                    : wave                      ? (int)e->W
                    : p->move == QMC_MOVE_ALL || group_sweeps(s, e->prec, e->W)
@@ -1740,7 +1751,9 @@ int qmc_ensemble_sweeps(qmc_ensemble* e, const qmc_sweep_params* p, double* e_su
     if (p->move == QMC_MOVE_SINGLE) {
       if ((rc = enqueue_single_sweeps(e, A, trace, e->st))) return rc;
     } else if (p->move == QMC_MOVE_DRIFT) {
-      if (tdd && e->prec == QMC_FP64)
+      if (hdd)
+        HIP_TRY(half_dd(s->d64, s->terms, e->view<double>(), A, e->partial, trace, e->st));
+      else if (tdd && e->prec == QMC_FP64)
         HIP_TRY(tile_dd<double>(s->d64, e->view<double>(), s->tile, A, e->partial, trace, e->st));
       else if (tdd)
         HIP_TRY(tile_dd<float>(s->d32, e->view<float>(), s->tile, A, e->partial, trace, e->st));
@@ -2686,13 +2699,15 @@ int isdmc_steps(const qmc_system* s, const qmc_isdmc_params* p, uint64_t seed, i
   const int nainv = nu * nu + nd * nd;
   const int64_t T_all = p->n_burnin + p->n_steps;
   // sweep partial rows: one per 64 walkers (register engine), per block of
-  // the lane-group engine or per walker (wave engine)
+  // the lane-group engine, per wavefront of the half-wave engine or per
+  // walker (wave engine)
   const bool wave = s->wave();
   const bool f64 = sizeof(T) == 8;
   // one-step launches: the lane groups' longer prologue pays for 16 lanes a
   // walker (CH4) only; H2 took 27.9 us per step with them, 27.7 without
   const bool group = f64 && group_sweeps(s, QMC_FP64, p->n_walkers) && s->gops->wpb <= 4;
-  const int nb = (int)(cap / DMC_BLOCK), sweep_bs = wave ? 1 : (group ? s->gops->wpb : 64),
+  const bool half = s->use_half(f64 ? QMC_FP64 : QMC_MIXED);
+  const int nb = (int)(cap / DMC_BLOCK), sweep_bs = half ? HALF_W : (wave ? 1 : (group ? s->gops->wpb : 64)),
             sweep_rows = (int)(cap / sweep_bs);
   // a stream of its own (graphs cannot capture the null stream) and the
   // two-step graphs, one per parity of the buffer a pair of steps starts in
@@ -2775,7 +2790,9 @@ int isdmc_steps(const qmc_system* s, const qmc_isdmc_params* p, uint64_t seed, i
     SweepArgs sa{1, (uint32_t)u, seed, 0, p->time_step, 0, p->max_drift};
     if (from_ctl) sa.step0_dev = &B.ctl->step;
     if constexpr (sizeof(T) == 8) {
-      if (wave)
+      if (half)
+        HIP_TRY(half_dd(s->d64, s->terms, V[c], sa, partial, nullptr, st));
+      else if (wave)
         HIP_TRY(wave_dd<double>(s->d64, V[c], s->shape(), sa, partial, nullptr, st));
       else if (group)
         HIP_TRY(s->gops->dd64_ns(s->d64, V[c], sa, partial, nullptr, st));
