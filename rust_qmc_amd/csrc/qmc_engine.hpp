@@ -300,7 +300,7 @@ __device__ __forceinline__ double jastrow_u(const DevSys<double>& S, const T ru[
 #pragma unroll
     for (int j = i + 1; j < N; ++j) {
       double dx = r[i][0] - r[j][0], dy = r[i][1] - r[j][1], dz = r[i][2] - r[j][2];
-      double rr = sqrt(dx * dx + dy * dy + dz * dz);
+      double rr = M<double>::dist(dx * dx + dy * dy + dz * dz);
       u += uee_val<double, Js>(S, rr, (i < NU) == (j < NU)) + S.cst_ee;
     }
   if (S.en_on)
@@ -308,7 +308,7 @@ __device__ __forceinline__ double jastrow_u(const DevSys<double>& S, const T ru[
     for (int i = 0; i < N; ++i)
       Bs::nuclei(S, [&](int I) {
         double dx = r[i][0] - S.nuc[I][0], dy = r[i][1] - S.nuc[I][1], dz = r[i][2] - S.nuc[I][2];
-        u += uen_val<double, Js>(S, sqrt(dx * dx + dy * dy + dz * dz), I);
+        u += uen_val<double, Js>(S, M<double>::dist(dx * dx + dy * dy + dz * dz), I);
       });
   return u;
 }

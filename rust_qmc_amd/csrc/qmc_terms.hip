@@ -7,6 +7,14 @@
 // Gauss-Jordan inversion, its AO derivatives against its inverse column and
 // its Jastrow partners, with 63 of 64 lanes busy and nothing but the rows
 // in transit, the positions and the sums over electrons in LDS.
+//
+// Measured for 8,192 benzene walkers, E_L with every derivative: 7,670 us
+// with a wavefront per walker, about 350 here; 1,003 evaluations 458 -> 105
+// us a call.  Cycles per wavefront: Slater rows 50 k, inversion 41 k,
+// determinant and nuclear terms 80 k, partners 11 k, parameters 20 k, for
+// about 10 k instructions: the latency of scalar loads (coefficient rows) and
+// of dependent FP64 instructions is what counts.  The rows from LDS were
+// slower (500 us a measure call against 402: the wider loads spill).
 #include "qmc_terms.hpp"
 
 #include <cstring>
