@@ -516,4 +516,14 @@ hipError_t terms_eval(const void* Sd, const TermTab* T, int64_t W, const double*
   return hipGetLastError();
 }
 
+hipError_t terms_eloc(const void* Sd, const TermTab* T, EnsView<double> E, hipStream_t st) {
+  TermArgs A{};
+  A.D.W = E.W;
+  A.D.pos64 = E.pos;
+  A.D.ld = E.ld;
+  A.O.eloc = E.eloc;
+  terms_kernel<false><<<(unsigned)((E.W + GW - 1) / GW), 128, 0, st>>>((const DevSys<double>*)Sd, T, A);
+  return hipGetLastError();
+}
+
 }  // namespace qmc

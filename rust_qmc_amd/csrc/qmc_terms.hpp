@@ -64,5 +64,7 @@ hipError_t terms_derivs(const void* Sd, const TermTab* T, DerivArgs A, hipStream
 // qmc_evaluate's outputs from [W][N][3] positions, in FP64
 hipError_t terms_eval(const void* Sd, const TermTab* T, int64_t W, const double* pos, EvalOut O, int* sing,
                       hipStream_t st);
+// E_L of an ensemble's walkers (its eloc) from their positions
+hipError_t terms_eloc(const void* Sd, const TermTab* T, EnsView<double> E, hipStream_t st);
 
 }  // namespace qmc
