@@ -1570,6 +1570,7 @@ int ensure_cap(double** p, size_t* cap, size_t n) {
   if (*cap >= n) return QMC_OK;
   if (*p) HIP_TRY(hipFree(*p));
   *p = nullptr;
+  *cap = 0;
   HIP_TRY(hipMalloc(p, n * sizeof(double)));
   *cap = n;
   return QMC_OK;
