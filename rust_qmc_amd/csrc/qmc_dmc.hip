@@ -5,11 +5,11 @@
 //   dmc_branch_kernel   copies m_w = min(floor(W_w + xi_w), 3) per walker with
 //                       W_w = exp(tau (E_ref - (E_L' + E_L) / 2)), and the
 //                       in-workgroup exclusive scan of m
-//   dmc_scan_kernel     one workgroup scans the workgroup totals, giving the
-//                       new population size (capped at the capacity)
-//   dmc_copy_kernel     writes every survivor and clone into buffer nxt in
-//                       source order (clones adjacent) with per-chunk sums of
-//                       E_L and of the HF force over the new population
+//   dmc_copy_kernel     scans the workgroup totals, giving the new population
+//                       size (capped at the capacity), and writes every
+//                       survivor and clone into buffer nxt in source order
+//                       (clones adjacent) with per-chunk sums of E_L and of
+//                       the HF force over the new population
 //   dmc_finalize_kernel mean E_L, population, force sums, the sweep's accepted
 //                       moves and the E_ref feedback
 //                       E_ref = <E_L> - damping ln(N / N_target) / tau
@@ -143,47 +143,17 @@ __global__ void __launch_bounds__(DMC_BLOCK) dmc_branch_kernel(DmcArgs a, DmcBuf
   if (threadIdx.x == DMC_BLOCK - 1) b.bsum[blockIdx.x] = (int64_t)(base + x);
 }
 
-__global__ void __launch_bounds__(1024) dmc_scan_kernel(DmcArgs a, DmcBufs b, int nxt, int nb) {
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  int64_t v[4], s = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = t * 4 + i;
-    v[i] = k < nb ? b.bsum[k] : 0;
-    s += v[i];
-  }
-  int64_t x = s;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int64_t y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  __shared__ int64_t wt[16];
-  if (lane == 63) wt[wv] = x;
-  __syncthreads();
-  int64_t base = 0;
-  for (int i = 0; i < wv; ++i) base += wt[i];
-  int64_t run = base + x - s;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = t * 4 + i;
-    if (k < nb) b.bsum[k] = run;
-    run += v[i];
-  }
-  if (t == 1023) {
-    const int64_t total = base + x;
-    const int64_t n = total < a.cap ? total : a.cap;
-    b.ctl->n_live[nxt] = n;
-    b.ctl->dropped += total - n;
-  }
-}
-
 // Compaction as a grid-stride loop over items (kind, chunk) of 256 source
 // walkers: kind 0 copies the scalar state and sums E_L over the copies,
 // kinds 1..n3+nainv copy one row of positions or inverse elements (one load,
 // c coalesced stores per walker), and with forces the n_nuc last kinds sum
 // c times the HF force on one nucleus.  Items exist only for the live
 // source population, so the work follows it rather than the capacity.
+// Each workgroup first scans the live chunks' totals into its LDS (at most
+// DMC_MAX_BLOCKS of them, one per thread up to 65,536 walkers; the sums stay
+// below 3 * 2^20) and workgroup 0 publishes the new population: a step is
+// bound by its small launches, and the same scan as a kernel of its own was
+// one of five (H2, 16,384 target walkers, whole run: 5,250 -> 5,000 us).
 template <class T>
 __global__ void __launch_bounds__(DMC_BLOCK) dmc_copy_kernel(const DevSys<double>* __restrict__ Sd, DmcArgs a,
                                                              DmcBufs b, int cur, EnsView<T> src, EnsView<T> dst,
@@ -196,6 +166,33 @@ __global__ void __launch_bounds__(DMC_BLOCK) dmc_copy_kernel(const DevSys<double
   const int64_t n_items = nch * (1 + rows + (with_force ? a.n_nuc : 0));
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   __shared__ double sh[DMC_BLOCK / 64][1 + 3 * MAXN];
+  __shared__ int off[DMC_MAX_BLOCKS], wt[DMC_BLOCK / 64];
+  {
+    // exclusive scan of bsum[0, nch): thread t takes per consecutive chunks
+    const int n = (int)nch, per = (n + DMC_BLOCK - 1) / DMC_BLOCK, k0 = (int)threadIdx.x * per;
+    int s = 0;
+    for (int k = k0; k < k0 + per && k < n; ++k) {
+      off[k] = s;
+      s += (int)b.bsum[k];
+    }
+    int x = s;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) wt[wv] = x;
+    __syncthreads();
+    int base = x - s;
+    for (int i = 0; i < wv; ++i) base += wt[i];
+    for (int k = k0; k < k0 + per && k < n; ++k) off[k] += base;
+    if (blockIdx.x == 0 && threadIdx.x == DMC_BLOCK - 1) {
+      const int64_t total = base + s, live = total < a.cap ? total : a.cap;
+      b.ctl->n_live[1 - cur] = live;
+      b.ctl->dropped += total - live;
+    }
+    __syncthreads();
+  }
   for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int kind = (int)(item / nch);
     const int64_t ch = item - (int64_t)kind * nch;
@@ -203,7 +200,7 @@ __global__ void __launch_bounds__(DMC_BLOCK) dmc_copy_kernel(const DevSys<double
     int c = 0;
     int64_t d0 = 0;
     if (w < W) {
-      d0 = b.bsum[ch] + b.loff[w];
+      d0 = off[ch] + b.loff[w];
       c = b.copies[w];
       if (d0 + c > a.cap) c = d0 < a.cap ? (int)(a.cap - d0) : 0;
     }
@@ -353,11 +350,10 @@ hipError_t dmc_branch_step(const void* Sd, const DmcArgs& a, const DmcBufs& b, i
   if (a.cap <= 0 || a.cap % DMC_BLOCK || a.cap / DMC_BLOCK > DMC_MAX_BLOCKS || a.n_nuc > MAXN || src.ld < a.cap ||
       dst.ld < a.cap)
     return hipErrorInvalidValue;
-  const int nb = (int)(a.cap / DMC_BLOCK), nxt = 1 - cur;
+  const int nb = (int)(a.cap / DMC_BLOCK);
   if (sweep_bs < 1 || (int64_t)sweep_nblk * sweep_bs < a.cap)  // the sweep's partial rows cover the capacity
     return hipErrorInvalidValue;
   dmc_branch_kernel<<<nb, DMC_BLOCK, 0, st>>>(a, b, cur, src.eloc, eprev_src, t);
-  dmc_scan_kernel<<<1, 1024, 0, st>>>(a, b, nxt, nb);
   dmc_copy_kernel<T><<<nb < 1024 ? nb : 1024, DMC_BLOCK, 0, st>>>((const DevSys<double>*)Sd, a, b, cur, src, dst,
                                                                   eprev_dst, with_force);
   dmc_finalize_kernel<<<1, 1024, 0, st>>>(a, b, cur, ts, with_force, sweep_part, sweep_bs, acc_out);

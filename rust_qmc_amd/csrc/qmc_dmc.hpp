@@ -13,7 +13,7 @@ namespace qmc {
 
 constexpr int DMC_BLOCK = 256;        // walkers per branching workgroup
 constexpr int DMC_MAX_CLONES = 3;     // MAX_CLONES, is_dmc.rs:43
-constexpr int DMC_MAX_BLOCKS = 4096;  // the single-workgroup scan covers 4 sums per thread
+constexpr int DMC_MAX_BLOCKS = 4096;  // the copy kernel scans their totals in LDS
 
 // device-resident control block of one DMC run
 struct DmcCtl {
@@ -45,7 +45,7 @@ struct DmcBufs {
   DmcCtl* ctl;
   int* copies;     // [cap]
   int* loff;       // [cap] in-block exclusive offsets
-  int64_t* bsum;   // [cap / DMC_BLOCK] block totals, then block offsets
+  int64_t* bsum;   // [cap / DMC_BLOCK] block totals
   double* part;    // [cap / DMC_BLOCK][1 + 3 * n_nuc]
   double* e_trace;    // [steps] mean E_L after branching
   double* pop_trace;  // [steps] population after branching

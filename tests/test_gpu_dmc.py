@@ -60,6 +60,20 @@ def test_isdmc_matched_branching_parity_fp64(Q, oracle, name):
     assert r.acceptance_rate == pytest.approx(ro["acceptance_rate"], rel=1e-12)
 
 
+@pytest.mark.parametrize("W", [255, 257, 65537])
+def test_isdmc_chunk_offsets(Q, oracle, W):
+    """Populations at the edge of a 256-walker chunk and past 256 chunks,
+    where a thread of the offset scan takes more than one chunk: the same
+    counts, and the same energies, which need every walker in its place.
+    The bound is the population test's."""
+    g, o = _pair(Q, oracle, "h2")
+    cap = 256 * ((2 * W + 255) // 256)
+    dmc, r, ro = _run_both(Q, g, o, 11, W, 4, 1, 0.02, n_eq=2, n_fs=50, capacity=cap)
+    assert np.array_equal(dmc.populations, ro["populations"])
+    assert _close(dmc.energies, ro["energies"], 1e-9)
+    assert r.dropped == ro["dropped"] == 0
+
+
 def test_isdmc_capacity_drops_match(Q, oracle):
     """Negative damping fills the capacity; the clones past it are dropped
     in source order exactly as the oracle drops them."""
