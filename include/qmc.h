@@ -182,11 +182,13 @@ int qmc_set_precision(qmc_system* sys, int32_t precision);
  * VGPRs (compiled electron counts up to 5 + 5); the wave engine keeps one
  * walker per wavefront in LDS (any count up to 32 per spin); the tile
  * engine moves 16 walkers per workgroup together with an MFMA MO
- * contraction (mixed-precision sweeps of 21 + 21-electron systems such as
- * benzene; state build, refresh and evaluation stay on the wave engine).
- * AUTO picks the register engine when it exists for the system, else the
- * tile engine for mixed-precision sweeps when it fits, else the wave
- * engine.  The register engine uses kernels specialised to the system's
+ * contraction (sweeps of 21 + 21-electron systems such as benzene).  AUTO
+ * picks the register engine when it exists for the system, else the tile
+ * engine when it fits, else the wave engine.  Under AUTO, FP64 work of few
+ * walkers of a compiled shell structure runs one electron per lane, and FP64
+ * benzene sweeps run with a walker on half a wavefront; evaluations and
+ * derivatives of benzene run one electron per lane unless WAVE is selected.
+ * The register engine uses kernels specialised to the system's
  * shell structure when one is compiled (H2, both Li atoms, CH4 STO-3G and
  * 6-31G); GENERIC forces its kernels with run-time shell loops. */
 #define QMC_ENGINE_AUTO 0
