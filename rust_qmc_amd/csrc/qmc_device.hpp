@@ -642,6 +642,13 @@ __device__ __forceinline__ void uen_d(const DevSys<T>& S, T r, T ir, int I, T& u
   lap = s2 * iD2 * iD2 - T(2) * S.b_en * ap * iD2 * iD + T(2) * u1 * ir;
 }
 
+// |a| as a candidate of a pivot search spread over lanes, where a NaN counts
+// as infinity: every lane then orders the candidates alike, each row is the
+// pivot of one column, and a row with a NaN makes the determinant NaN.
+// (Plain comparisons skip a NaN row until only used rows are left, and one
+// of those then serves twice with a finite pivot.)
+__device__ __forceinline__ double pivot_mag(double a) { return fmin(fabs(a), INFINITY); }
+
 // ---------------------------------------------------------------------------
 // Gauss-Jordan inversion with partial pivoting, fully register resident
 // (row swaps by selects).  Returns ln|det| and sign; a singular matrix

@@ -185,7 +185,7 @@ __device__ __forceinline__ void group_invert(Lds& L, int lane, int base, int slo
 #pragma unroll
   for (int c = 0; c < NS; ++c) {
     const bool act = even || c < ns;
-    const double v = used ? -1.0 : fabs(a[c]);
+    const double v = used ? -1.0 : pivot_mag(a[c]);
     double best = -2.0;
     int p = 0;
 #pragma unroll

@@ -232,10 +232,10 @@ __global__ void __launch_bounds__(TILE_T, 2) tile_invert_kernel(const DevSys<dou
     double* pr_l = prow + wt * NS;
 #pragma unroll
     for (int c = 0; c < NS; ++c) {
-      double best = used0 ? -1.0 : fabs(r0[c]);
+      double best = used0 ? -1.0 : pivot_mag(r0[c]);
       int p = g;
       if (!used1) {
-        const double v = fabs(r1[c]);
+        const double v = pivot_mag(r1[c]);
         if (v > best) {
           best = v;
           p = g + 16;

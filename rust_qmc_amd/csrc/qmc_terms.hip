@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(128, 2) terms_kernel(const DevSys<double>* __r
   int mine = 0;
 #pragma unroll
   for (int c = 0; c < NS; ++c) {
-    L.colv[sp][grp][slot] = used ? -1.0 : fabs(a[c]);
+    L.colv[sp][grp][slot] = used ? -1.0 : pivot_mag(a[c]);
     wave_sync();
     double best = -2.0;
     int p = 0;
