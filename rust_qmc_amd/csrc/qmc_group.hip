@@ -521,8 +521,8 @@ __global__ void __launch_bounds__(64) group_derivs_kernel(const DevSys<double>* 
     om[c][1] -= sy;
     om[c][2] -= sz;
   };
-  double gd[3];
-  const double ei = group_energy<Bs>(S, x, y, z, wgt, P, on_shell, gd);
+  double gd[3], lap;
+  const double ei = group_energy<Bs>(S, x, y, z, wgt, P, on_shell, gd, lap);
   Bs::nuclei(S, [&](int I) {
     const double dx = x - S.nuc[I][0], dy = y - S.nuc[I][1], dz = z - S.nuc[I][2];
     double rr, ir;
@@ -667,8 +667,8 @@ __global__ void __launch_bounds__(64) group_eval_kernel(const DevSys<double>* __
     for (int m = 0; m < NS; ++m) v += mo[ao * 2 * Sh::NSP + m] * col[m];
     return v;
   };
-  double gd[3];
-  const double ei = group_energy<Bs>(S, x, y, z, wgt, P, NoShell{}, gd);
+  double gd[3], lap;
+  const double ei = group_energy<Bs>(S, x, y, z, wgt, P, NoShell{}, gd, lap);
   const double el = gsum<G>(elec ? ei : 0.0) + S.vnn, gs = S.grad_scale;
   if (live && g == 0 && O.eloc) O.eloc[w] = el;
   if (live && elec) {
@@ -678,7 +678,7 @@ __global__ void __launch_bounds__(64) group_eval_kernel(const DevSys<double>* __
       q[1] = gd[1] + gs * P.gy;
       q[2] = gd[2] + gs * P.gz;
     }
-    if (O.lap) O.lap[w * N + e] = 2.0 * (P.v - ei);  // ei = -lap / 2 + v
+    if (O.lap) O.lap[w * N + e] = lap;
   }
 }
 

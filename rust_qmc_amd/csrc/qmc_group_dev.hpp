@@ -148,22 +148,22 @@ __device__ __forceinline__ PairSums group_pairs(const DevSys<double>& S, const L
 
 // -1/2 lap psi / psi of one electron plus its potential share, from the
 // determinant terms of its weights and its pair sums (electron_terms);
-// on_shell as det_terms_w, gd receives grad D / D
+// on_shell as det_terms_w, gd receives grad D / D and lap the Laplacian
 template <class Bs, class Wgt, class OnShell>
 __device__ __forceinline__ double group_energy(const DevSys<double>& S, double x, double y, double z, Wgt wgt,
-                                               const PairSums& P, OnShell on_shell, double gd[3]) {
+                                               const PairSums& P, OnShell on_shell, double gd[3], double& lap) {
   double ld;
   det_terms_w<double, Wgt, OnShell, Bs>(S, x, y, z, wgt, gd[0], gd[1], gd[2], ld, on_shell);
   const double gs = S.grad_scale;
   const double lj = (S.flags & F_J2_LAP_QUIRK) ? P.lap + P.sq : P.lap + P.gx * P.gx + P.gy * P.gy + P.gz * P.gz;
-  const double lap = ld + lj + 2.0 * gs * (gd[0] * P.gx + gd[1] * P.gy + gd[2] * P.gz);
+  lap = ld + lj + 2.0 * gs * (gd[0] * P.gx + gd[1] * P.gy + gd[2] * P.gz);
   return -0.5 * lap + P.v;
 }
 template <class Bs, class Wgt>
 __device__ __forceinline__ double group_energy(const DevSys<double>& S, double x, double y, double z, Wgt wgt,
                                                const PairSums& P) {
-  double gd[3];
-  return group_energy<Bs>(S, x, y, z, wgt, P, NoShell{}, gd);
+  double gd[3], lap;
+  return group_energy<Bs>(S, x, y, z, wgt, P, NoShell{}, gd, lap);
 }
 
 // Both sectors' Slater matrices inverted at once, one row (electron) per

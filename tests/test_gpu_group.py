@@ -153,3 +153,28 @@ def test_singular_configuration_is_reported(Q):
     s.set_flags(Q.QMC_FLAGS_REFERENCE)
     o = s.evaluate_batch(pos)
     assert o["logabs"][4] == -np.inf and o["sign"][4] == 0.0 and np.isfinite(o["logabs"][:4]).all()
+
+
+@pytest.mark.parametrize("distance", [0.0, 1e-9, 1e-4])
+@pytest.mark.parametrize("name", ["li", "ch4-sto3g", "ch4-631g"])
+def test_laplacian_next_to_a_nucleus_or_an_electron(Q, name, distance):
+    """Where 1/r is many orders larger than the Laplacian, the Laplacian keeps
+    its own digits: electron 0 at a nucleus, and the last electron on electron
+    1, against the one-walker-per-lane kernel (1e-9 of the finite values'
+    scale, as above)."""
+    s = {"li": lambda: Q.Lithium(0), "ch4-sto3g": lambda: Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0),
+         "ch4-631g": lambda: Q.MethaneGTO()}[name]()
+    rng = np.random.default_rng(9)
+    pos = 0.8 * rng.normal(size=(5, s.n_elec, 3))
+    R, d = s.get_nuclei(), distance * np.array([2.0, -1.0, 2.0]) / 3.0
+    for w in range(4):
+        pos[w, 0] = R[w % len(R)] + d
+    pos[4, -1] = pos[4, 1] + d
+    res = []
+    for engine in ("auto", "register"):
+        s.set_engine(engine)
+        res.append(s.evaluate_batch(pos, ("lap",))["lap"])
+    ok = np.isfinite(res[1])
+    assert np.array_equal(np.isfinite(res[0]), ok) and ok[4].all()
+    for a, b, k in zip(*res, ok):
+        assert np.abs(a - b)[k].max() <= 1e-9 * max(1.0, np.abs(b[k]).max())
