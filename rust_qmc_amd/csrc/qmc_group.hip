@@ -31,13 +31,15 @@ __global__ void __launch_bounds__(64) group_ae_kernel(const DevSys<double>* __re
   constexpr int N = Sh::N, NS = Sh::NS, G = Sh::G, WPB = Sh::WPB;
   __shared__ typename Sh::Lds L;
   const DevSys<double>& S = *Sp;
+  const int64_t blk = (int64_t)blockIdx.y * gridDim.x + blockIdx.x, nblk = (E.W + WPB - 1) / WPB;
+  if (blk >= nblk) return;
   group_fill_mo<NU, ND, Bs>(S, L);
   const int lane = threadIdx.x, grp = lane / G, g = lane % G;
   const bool elec = g < N;
   const int sp = elec && g >= NU ? 1 : 0, slot = elec ? g - (sp ? NU : 0) : 0, ns = sp ? ND : NU;
   const int base = grp * G + (sp ? NU : 0);  // first lane of this lane's sector
   const int e = S.sector_elec[sp][slot];
-  const int64_t w = (int64_t)blockIdx.x * WPB + grp;
+  const int64_t w = blk * WPB + grp;
   const bool live = w < E.W;
   const int64_t wl = live ? w : E.W - 1;  // walkers past the end shadow the last one and write nothing
   T r[3];
@@ -100,7 +102,7 @@ __global__ void __launch_bounds__(64) group_ae_kernel(const DevSys<double>* __re
     if (el_trace && head) el_trace[(int64_t)s * A.trace_ld + w] = el;
     const double e1 = wsum(head ? el : 0.0), e2 = wsum(head ? el * el : 0.0), na = wsum(head && acc ? 1.0 : 0.0);
     if (lane == 0) {
-      double* p = partial + ((int64_t)s * gridDim.x + blockIdx.x) * 3;
+      double* p = partial + ((int64_t)s * nblk + blk) * 3;
       p[0] = e1;
       p[1] = e2;
       p[2] = na;
@@ -687,9 +689,12 @@ __global__ void __launch_bounds__(64) group_eval_kernel(const DevSys<double>* __
 // ---------------------------------------------------------------------------
 template <int NU, int ND, class Bs, class Js, class T>
 static hipError_t launch_ae(const void* Sd, EnsView<T> E, SweepArgs A, double* partial, double* trace, hipStream_t st) {
+  // rows of at most 65,536 workgroups: a walker takes up to 16 lanes, and a
+  // grid dimension holds fewer than 2^32 of them
   constexpr int wpb = GroupShape<NU, ND, Bs>::WPB;
-  group_ae_kernel<NU, ND, Bs, Js, T><<<(unsigned)((E.W + wpb - 1) / wpb), 64, 0, st>>>((const DevSys<double>*)Sd, E, A,
-                                                                                     partial, trace);
+  const int64_t nblk = (E.W + wpb - 1) / wpb, x = nblk < 65536 ? nblk : 65536;
+  const dim3 grid((unsigned)x, (unsigned)((nblk + x - 1) / x));
+  group_ae_kernel<NU, ND, Bs, Js, T><<<grid, 64, 0, st>>>((const DevSys<double>*)Sd, E, A, partial, trace);
   return hipGetLastError();
 }
 

@@ -1,0 +1,36 @@
+"""Ensembles and batches past the limits at which launches, staging buffers
+and scratch are divided: nothing may change at a seam."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def Q():
+    import rust_qmc_amd
+
+    return rust_qmc_amd
+
+
+def test_all_electron_past_one_row_of_workgroups(Q):
+    """65,536 workgroups of four CH4 walkers are one row of the grid: the
+    walkers around its end move as the wave engine moves them."""
+    s = Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0, precision="mixed")
+    W = 4 * 65536 + 6
+    out = []
+    for engine in ("auto", "wave"):
+        s.set_engine(engine)
+        ens = Q.Ensemble(s, W, 3)
+        p0 = ens.positions()
+        es, _, acc = ens.sweeps(2, 0.2, move=Q.QMC_MOVE_ALL)
+        out.append((acc, ens.positions(), ens.state()[2], es))
+    (acc, pos, el, es), (acc_w, pos_w, _, _) = out
+    assert np.array_equal(acc, acc_w)
+    np.testing.assert_array_equal(pos, pos_w)
+    np.testing.assert_allclose(es[-1], el.sum(), rtol=1e-11)  # every partial sum counted once
+    # E_L of the walkers that moved is FP64 at the FP32 positions; 1e-8 leaves
+    # FP64 rounding a factor of 1e7 for the worst-conditioned Slater matrix
+    moved = (pos != p0).any(axis=(1, 2))
+    ref = Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0).evaluate_batch(pos[moved], ("eloc",))["eloc"]
+    np.testing.assert_allclose(el[moved], ref, rtol=1e-8, atol=1e-8)
