@@ -1731,23 +1731,28 @@ int qmc_ensemble_sweeps(qmc_ensemble* e, const qmc_sweep_params* p, double* e_su
   // drift-diffusion moves on the tile engine where it runs single-electron
   // sweeps; all-electron moves on the wave engine (also for tile-engine
   // systems): one block per walker
-  const bool hdd = p->move == QMC_MOVE_DRIFT && s->use_half(e->prec);
+  const bool half = sm && s->use_half(e->prec);
+  const bool group = !wave && (!sm || group_sweeps(s, e->prec, e->W));
+  const bool hdd = p->move == QMC_MOVE_DRIFT && half;
   const bool tdd = p->move == QMC_MOVE_DRIFT && !hdd && s->tile_dd(e->prec);
   const int nblk = p->move == QMC_MOVE_SINGLE ? (int)sweep_blocks(e)
                    : hdd                       ? (int)half_blocks(e->W)
                    : tdd                       ? (int)tile_blocks(e->W)
                    : wave                      ? (int)e->W
-                   : p->move == QMC_MOVE_ALL || group_sweeps(s, e->prec, e->W)
-                       ? (int)group_blocks(s, e->W)
-                       : (int)((e->W + 63) / 64);
+                   : group                     ? (int)group_blocks(s, e->W)
+                                               : (int)((e->W + 63) / 64);
   const int refresh = p->refresh_interval > 0 ? p->refresh_interval : 0;
-  // sweeps per launch: 64 unless their partial sums would pass 32 MiB, then
-  // down to 16.  Each launch loads and stores the state and is followed by a
-  // reduction: 64 instead of 16 took H2's all-electron step from 3.5 to
-  // 3.0 us, 256 CH4 sweeps of 65,536 walkers from 7.14 to 7.00 ms.
-  int chunk = p->steps_per_launch > 0
-                  ? p->steps_per_launch
-                  : (int)std::min<int64_t>(64, std::max<int64_t>(16, (32 << 20) / (24 * (int64_t)nblk)));
+  // Sweeps per launch: 64 by default, or what the caller asks for, or fewer
+  // so that their partial sums stay within 32 MiB or, where that is more,
+  // what 16 sweeps (the caller's number) need with a row per 64 walkers
+  // (per tile of 16 for the half-wave engine), as coarse as rows can be.
+  // Each launch loads and stores the state and is followed by a reduction:
+  // 64 instead of 16 took H2's all-electron step from 3.5 to 3.0 us, 256
+  // CH4 sweeps of 65,536 walkers from 7.14 to 7.00 ms.
+  const int want = p->steps_per_launch > 0 ? p->steps_per_launch : 64;
+  const int64_t coarse = half ? tile_blocks(e->W) : group ? (e->W + 63) / 64 : nblk,
+                room = std::max<int64_t>(32 << 20, 24 * coarse * (p->steps_per_launch > 0 ? want : 16));
+  const int chunk = (int)std::min<int64_t>(want, std::max<int64_t>(1, room / (24 * (int64_t)nblk)));
   if ((rc = ensure_cap(&e->partial, &e->partial_cap, (size_t)chunk * nblk * 3))) return rc;
   if ((rc = ensure_cap(&e->sums, &e->sums_cap, (size_t)p->n_steps * 3))) return rc;
   Staged tr;
@@ -1784,7 +1789,7 @@ int qmc_ensemble_sweeps(qmc_ensemble* e, const qmc_sweep_params* p, double* e_su
         HIP_TRY(wave_dd<double>(s->d64, e->view<double>(), s->shape(), A, e->partial, trace, e->st));
       else if (wave)
         HIP_TRY(wave_dd<float>(s->d32, e->view<float>(), s->shape(), A, e->partial, trace, e->st));
-      else if (group_sweeps(s, e->prec, e->W))
+      else if (group)
         HIP_TRY(s->gops->dd64_ns(s->d64, e->view<double>(), A, e->partial, trace, e->st));
       else if (e->prec == QMC_FP64)
         HIP_TRY((s->no_series() ? s->ops->dd64_ns : s->ops->dd64)(s->d64, e->view<double>(), A, e->partial, trace,

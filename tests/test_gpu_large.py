@@ -34,3 +34,18 @@ def test_all_electron_past_one_row_of_workgroups(Q):
     moved = (pos != p0).any(axis=(1, 2))
     ref = Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0).evaluate_batch(pos[moved], ("eloc",))["eloc"]
     np.testing.assert_allclose(el[moved], ref, rtol=1e-8, atol=1e-8)
+
+
+@pytest.mark.parametrize("asked", [0, 16, 40])
+def test_partial_sums_of_a_large_ensemble_stay_bounded(Q, asked):
+    """All-electron CH4 moves have a partial-sum row per four walkers; a launch
+    takes as many steps as 32 MiB of them hold."""
+    s = Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0, precision="mixed")
+    W, n = 500_000, 40
+    ens = Q.Ensemble(s, W, 3)
+    ens.set_timing()
+    es, _, acc = ens.sweeps(n, 0.2, move=Q.QMC_MOVE_ALL, steps_per_launch=asked)
+    per = (32 << 20) // (24 * (W // 4))
+    assert ens.timing()[1] == -(-n // per)
+    np.testing.assert_allclose(es[-1], ens.state()[2].sum(), rtol=1e-11)
+    assert (0 < acc).all() and (acc < W).all()
