@@ -1576,6 +1576,49 @@ int ensure_cap(double** p, size_t* cap, size_t n) {
   return QMC_OK;
 }
 
+struct DevFree {
+  void operator()(double* p) const { (void)hipFree(p); }
+};
+using DevBlock = std::unique_ptr<double, DevFree>;
+
+// The walkers' positions to (OUT) or from the caller's [W][n3], which may be
+// on the host: then through a device block of at most 32 MiB, so that the
+// call needs no room of the ensemble's own size, and less of it where even
+// that cannot be had.  The block is the caller's to free, after the stream
+// has drained.
+template <class T, bool OUT>
+int move_positions(const qmc_ensemble* e, int n3, double* user, DevBlock* block) {
+  T* pos = (T*)e->pos;
+  if (is_device_ptr(user)) {
+    if (OUT)
+      HIP_TRY(positions_out(pos, e->ld, e->W, n3, user, e->st));
+    else
+      HIP_TRY(positions_in(user, e->ld, e->W, e->ld, n3, pos, e->st));
+    return QMC_OK;
+  }
+  const size_t row = sizeof(double) * n3;
+  int64_t step = std::min<int64_t>(e->ld, (32 << 20) / row / 64 * 64);
+  double* dev = nullptr;
+  while (hipMalloc(&dev, row * step) != hipSuccess) {
+    if (step <= 64) return fail(QMC_ERR_HIP, "no device memory for 64 walkers' positions");
+    (void)hipGetLastError();
+    step = step / 2 / 64 * 64;
+  }
+  block->reset(dev);
+  for (int64_t w = 0; w < e->W; w += step) {
+    const int64_t n = std::min(step, e->W - w);
+    double* u = user + w * n3;
+    if (OUT) {
+      HIP_TRY(positions_out(pos + w, e->ld, n, n3, dev, e->st));
+      HIP_TRY(hipMemcpyAsync(u, dev, row * n, hipMemcpyDeviceToHost, e->st));
+    } else {
+      HIP_TRY(hipMemcpyAsync(dev, u, row * n, hipMemcpyHostToDevice, e->st));
+      HIP_TRY(positions_in(dev, e->ld, n, w + n == e->W ? e->ld - w : n, n3, pos + w, e->st));
+    }
+  }
+  return QMC_OK;
+}
+
 // blocks (partial-sum rows) of one single-electron sweep launch of e
 int64_t sweep_blocks(const qmc_ensemble* e) {
   const qmc_system* s = e->sys;
@@ -1663,31 +1706,22 @@ int qmc_ensemble_get_positions(const qmc_ensemble* e, double* pos) {
       }
     return QMC_OK;
   }
-  int rc, flag = 0;
-  CallBuffers B(e->st);
-  B.flag();
-  const int P = B.output(pos, sizeof(double) * n);
-  if ((rc = B.open())) return rc;
-  if (e->prec == QMC_FP64)
-    HIP_TRY(positions_out((const double*)e->pos, e->ld, e->W, n3, B.get<double>(P), e->st));
-  else
-    HIP_TRY(positions_out((const float*)e->pos, e->ld, e->W, n3, B.get<double>(P), e->st));
-  return B.close(&flag);
+  DevBlock block;
+  if (int rc = e->prec == QMC_FP64 ? move_positions<double, true>(e, n3, pos, &block)
+                                   : move_positions<float, true>(e, n3, pos, &block))
+    return rc;
+  HIP_TRY(hipStreamSynchronize(e->st));
+  return QMC_OK;
 }
 
 int qmc_ensemble_set_positions(qmc_ensemble* e, const double* pos) {
   if (!e || !pos) return fail(QMC_ERR_INVALID, "bad arguments");
   const int n3 = 3 * e->sys->h.n_elec();
-  int rc;
-  CallBuffers B(e->st);
-  const int P = B.input(pos, sizeof(double) * e->W * n3);
-  B.flag();
-  if ((rc = B.open())) return rc;
-  if (e->prec == QMC_FP64)
-    HIP_TRY(positions_in(B.get<double>(P), e->ld, e->W, n3, (double*)e->pos, e->st));
-  else
-    HIP_TRY(positions_in(B.get<double>(P), e->ld, e->W, n3, (float*)e->pos, e->st));
-  if ((rc = ens_refresh(e, 1))) return rc;
+  double* p = const_cast<double*>(pos);
+  DevBlock block;
+  int rc = e->prec == QMC_FP64 ? move_positions<double, false>(e, n3, p, &block)
+                               : move_positions<float, false>(e, n3, p, &block);
+  if (rc || (rc = ens_refresh(e, 1))) return rc;
   HIP_TRY(hipStreamSynchronize(e->st));
   return QMC_OK;
 }

@@ -7,10 +7,11 @@
 
 namespace qmc {
 
+// the first n walkers of pos; out holds [n][n3]
 template <class T>
-hipError_t positions_out(const T* pos, int64_t ld, int64_t W, int n3, double* out, hipStream_t st);
-// columns W .. ld of pos are set to zero
+hipError_t positions_out(const T* pos, int64_t ld, int64_t n, int n3, double* out, hipStream_t st);
+// likewise; the columns n .. nz of pos (nz >= n) are set to zero
 template <class T>
-hipError_t positions_in(const double* in, int64_t ld, int64_t W, int n3, T* pos, hipStream_t st);
+hipError_t positions_in(const double* in, int64_t ld, int64_t n, int64_t nz, int n3, T* pos, hipStream_t st);
 
 }  // namespace qmc

@@ -49,3 +49,36 @@ def test_partial_sums_of_a_large_ensemble_stay_bounded(Q, asked):
     assert ens.timing()[1] == -(-n // per)
     np.testing.assert_allclose(es[-1], ens.state()[2].sum(), rtol=1e-11)
     assert (0 < acc).all() and (acc < W).all()
+
+
+def _system(Q, name, precision):
+    return {"h2": lambda: Q.H2MoleculeMO(precision=precision), "ch4": lambda: Q.MethaneGTO(precision=precision),
+            "benzene": lambda: Q.BenzeneGTO(precision=precision)}[name]()
+
+
+# 1, 64 and 65 walkers; 512 KiB (10,922 of H2's 48 bytes, 2,184 of CH4's 240, 520
+# of benzene's 1,008) and 32 MiB (699,008 walkers of H2, 139,776 of CH4, 33,280
+# of benzene) are where the way of the copy changes
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("name,W", [("h2", 1), ("h2", 65), ("h2", 10_922), ("h2", 10_923), ("h2", 699_008), ("h2", 699_010),
+                                    ("ch4", 64), ("ch4", 2_185), ("ch4", 139_777 + 64), ("benzene", 65),
+                                    ("benzene", 521), ("benzene", 33_281)])
+def test_positions_round_trip(Q, name, W, precision):
+    """Positions set from the host and from the device come back exactly
+    (rounded to FP32 in mixed precision), and the state is theirs."""
+    s = _system(Q, name, precision)
+    n, rng = s.n_elec, np.random.default_rng(W)
+    pos = s.get_nuclei()[np.arange(n) % s.n_nuc] + rng.normal(size=(W, n, 3))
+    want = pos if precision == "fp64" else pos.astype(np.float32).astype(np.float64)
+    ens = Q.Ensemble(s, W, 1)
+    ens.set_positions(pos)
+    np.testing.assert_array_equal(ens.positions(), want)
+    some = np.unique(np.r_[0, W // 2, W - 1])
+    ref = s.evaluate_batch(want[some])
+    np.testing.assert_allclose(ens.state()[0][some], ref["logabs"], rtol=1e-9, atol=1e-9)
+    with Q.DeviceBuffer(pos.nbytes) as buf:
+        buf.upload(pos[::-1])
+        Q.check(Q.lib().qmc_ensemble_set_positions(ens._h, buf.ptr))
+        np.testing.assert_array_equal(ens.positions(), want[::-1])
+        Q.check(Q.lib().qmc_ensemble_get_positions(ens._h, buf.ptr))
+        np.testing.assert_array_equal(buf.download(np.float64, pos.size).reshape(pos.shape), want[::-1])
