@@ -1529,6 +1529,26 @@ bool tile_refresh_on() {
 
 int ensure_cap(double** p, size_t* cap, size_t n);
 
+// the tile refresh in parts of 65,536 walkers, which share 462 MB of Slater
+// rows (4,096 workgroups of the inversion are eight rounds of the chip)
+constexpr int64_t REFRESH_W = 65536;
+template <class T>
+int refresh_tiles(const qmc_ensemble* e) {
+  const qmc_system* s = e->sys;
+  for (int64_t w = 0; w < e->W; w += REFRESH_W) {
+    EnsView<T> E = e->view<T>();
+    E.W = std::min(REFRESH_W, e->W - w);
+    E.pos += w;
+    E.ainv += w;
+    E.logdet += w;
+    E.sign += w;
+    E.ju += w;
+    E.eloc += w;
+    HIP_TRY(tile_refresh<T>(s->d64, E, s->tile, e->rwork, nullptr, e->st));
+  }
+  return QMC_OK;
+}
+
 int ens_refresh(qmc_ensemble* e, int want_eloc) {
   const qmc_system* s = e->sys;
   // with E_L (a new ensemble, positions, parameters or nuclei) FP64 walkers
@@ -1537,7 +1557,7 @@ int ens_refresh(qmc_ensemble* e, int want_eloc) {
   const bool eloc64 = want_eloc && e->prec == QMC_FP64 && s->use_terms();
   bool tile = s->wave() && (!want_eloc || eloc64) && s->tile.ok && tile_refresh_on();
   if (tile) {
-    const int rc = ensure_cap(&e->rwork, &e->rwork_cap, tile_refresh_work(e->W));
+    const int rc = ensure_cap(&e->rwork, &e->rwork_cap, tile_refresh_work(std::min(REFRESH_W, e->W)));
     if (rc && !eloc64) return rc;
     if (rc) {  // no room for the Slater rows: the wave build needs none
       (void)hipGetLastError();
@@ -1545,10 +1565,7 @@ int ens_refresh(qmc_ensemble* e, int want_eloc) {
     }
   }
   if (tile) {
-    if (e->prec == QMC_FP64)
-      HIP_TRY(tile_refresh<double>(s->d64, e->view<double>(), s->tile, e->rwork, nullptr, e->st));
-    else
-      HIP_TRY(tile_refresh<float>(s->d64, e->view<float>(), s->tile, e->rwork, nullptr, e->st));
+    if (const int rc = e->prec == QMC_FP64 ? refresh_tiles<double>(e) : refresh_tiles<float>(e)) return rc;
     if (eloc64) HIP_TRY(terms_eloc(s->d64, s->terms, e->view<double>(), e->st));
   } else if (s->wave()) {
     if (e->prec == QMC_FP64)

@@ -82,3 +82,21 @@ def test_positions_round_trip(Q, name, W, precision):
         np.testing.assert_array_equal(ens.positions(), want[::-1])
         Q.check(Q.lib().qmc_ensemble_get_positions(ens._h, buf.ptr))
         np.testing.assert_array_equal(buf.download(np.float64, pos.size).reshape(pos.shape), want[::-1])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_benzene_refresh_in_parts(Q, precision):
+    """The tile refresh takes 65,536 walkers at a time: ln|psi| after it, and
+    E_L of one sweep from its inverses, are those of the positions on both
+    sides of the seam (1e-9 in FP64, the engines' bound; mixed: the FP32 E_L's
+    2e-4 + 1e-2 Ha)."""
+    s = _system(Q, "benzene", precision)
+    W = 65536 + 21
+    ens = Q.Ensemble(s, W, 2)
+    some = np.r_[0:8, 65536 - 8 : W]
+    ens.sweeps(2, 0.2, refresh_interval=2)  # the inverses are refreshed after the second sweep
+    ref = s.evaluate_batch(ens.positions()[some])
+    np.testing.assert_allclose(ens.state()[0][some], ref["logabs"], rtol=1e-9, atol=1e-9)
+    el = ens.sweeps(1, 0.2, refresh_interval=0, trace=True)[3][0][some]
+    ref = s.evaluate_batch(ens.positions()[some], ("eloc",))["eloc"]
+    np.testing.assert_allclose(el, ref, rtol=1e-9 if precision == "fp64" else 2e-4, atol=1e-9 if precision == "fp64" else 1e-2)
