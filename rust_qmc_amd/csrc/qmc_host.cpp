@@ -587,12 +587,13 @@ int64_t group_blocks(const qmc_system* s, int64_t W) { return (W + s->gops->wpb 
 // kernel for the 21 + 21-electron systems it fits, else the wave derivative
 // kernel when the wave or tile engine runs the system (or
 // its MO coefficients follow the geometry), else the register kernels.
-int launch_derivs(const qmc_system* s, DerivArgs A, int32_t prec, hipStream_t st) {
+// Wcall is the walker count of the whole call where A holds a part of it.
+int launch_derivs(const qmc_system* s, DerivArgs A, int64_t Wcall, int32_t prec, hipStream_t st) {
   if (s->use_terms()) {
     HIP_TRY(terms_derivs(s->d64, s->terms, A, st));
     return QMC_OK;
   }
-  if (group_fits(s, A.W, &GroupOps::w_deriv)) {
+  if (group_fits(s, Wcall, &GroupOps::w_deriv)) {
     HIP_TRY(s->gops->derivs_ns(s->d64, A, st));
     return QMC_OK;
   }
@@ -1355,11 +1356,9 @@ int qmc_local_energy(const qmc_system* s, int64_t W, const double* pos, double* 
 
 static_assert(3 * MAXN <= (int)(sizeof(DerivUnpack::fnn) / sizeof(double)), "fnn holds 3 MAXN forces");
 
-int qmc_derivatives(const qmc_system* sys, int64_t W, const double* pos, double* eloc, double* O, double* dE,
-                    double* F, double* Om, void* stream) {
-  if (!sys || !pos || W < 0) return fail(QMC_ERR_INVALID, "bad arguments");
-  if (W == 0) return QMC_OK;
-  hipStream_t st = (hipStream_t)stream;
+// qmc_derivatives of W configurations, a part of a call for Wcall
+static int derivatives_part(const qmc_system* sys, int64_t Wcall, int64_t W, const double* pos, double* eloc, double* O,
+                            double* dE, double* F, double* Om, hipStream_t st) {
   const int N = sys->h.n_elec();
   const Cols C(sys->h);
   int rc, flag = 0;
@@ -1378,7 +1377,7 @@ int qmc_derivatives(const qmc_system* sys, int64_t W, const double* pos, double*
             iY = h.empty() ? B.scratch(w8 * C.Qp) : B.output(h.data(), w8 * C.Qp);
   if ((rc = B.open())) return rc;
   DerivArgs A{W, C.P, C.M, C.Qp, B.get<double>(P), nullptr, nullptr, 0, B.get<double>(iY), W};
-  if ((rc = launch_derivs(sys, A, sys->precision, st))) return rc;
+  if ((rc = launch_derivs(sys, A, Wcall, sys->precision, st))) return rc;
   if (h.empty()) {
     DerivUnpack U{W, C.P, C.M, A.Y, B.get<double>(iE), B.get<double>(iO), B.get<double>(iD), B.get<double>(iF),
                   B.get<double>(iM), {}};
@@ -1403,6 +1402,21 @@ int qmc_derivatives(const qmc_system* sys, int64_t W, const double* pos, double*
   if ((rc = put(eloc, h.data() + (size_t)C.e() * W, W)) || (rc = put(O, o.data(), o.size())) ||
       (rc = put(dE, d.data(), d.size())) || (rc = put(F, f.data(), f.size())) || (rc = put(Om, om.data(), om.size())))
     return rc;
+  return QMC_OK;
+}
+
+int qmc_derivatives(const qmc_system* sys, int64_t W, const double* pos, double* eloc, double* O, double* dE,
+                    double* F, double* Om, void* stream) {
+  if (!sys || !pos || W < 0) return fail(QMC_ERR_INVALID, "bad arguments");
+  // parts of 131,072 configurations (a few hundred MB with the unpacked
+  // outputs), many rounds of any derivative kernel
+  const int64_t step = 131072;
+  const int n3 = 3 * sys->h.n_elec(), P = sys->h.n_params(), M3 = 3 * sys->h.n_nuc();
+  const auto at = [](double* p, int64_t n) { return p ? p + n : nullptr; };
+  for (int64_t w = 0; w < W; w += step)
+    if (const int rc = derivatives_part(sys, W, std::min(step, W - w), pos + w * n3, at(eloc, w), at(O, w * P),
+                                        at(dE, w * P), at(F, w * M3), at(Om, w * M3), (hipStream_t)stream))
+      return rc;
   return QMC_OK;
 }
 
@@ -1438,7 +1452,7 @@ int qmc_derivatives_noalloc(const qmc_system* sys, int64_t W, const double* pos,
   HIP_TRY(noalloc_scratch(&Y));
   hipStream_t st = (hipStream_t)stream;
   DerivArgs A{W, C.P, C.M, C.Qp, pos, nullptr, nullptr, 0, Y, W};
-  if (int rc = launch_derivs(sys, A, sys->precision, st)) return rc;
+  if (int rc = launch_derivs(sys, A, W, sys->precision, st)) return rc;
   DerivUnpack U{W, C.P, C.M, Y, eloc, O, dE, F, Om, {}};
   hf_nn_fill(sys->h, U.fnn);
   HIP_TRY(launch_deriv_unpack(U, st));
@@ -1911,7 +1925,7 @@ int qmc_ensemble_measure(qmc_ensemble* e, int32_t reset) {
     A.pos64 = (const double*)e->pos;
   else
     A.pos32 = (const float*)e->pos;
-  if ((rc = launch_derivs(s, A, e->prec, e->st))) return rc;
+  if ((rc = launch_derivs(s, A, e->W, e->prec, e->st))) return rc;
   if (e->ld > e->W)  // the Gram reads the padding columns (up to W rounded to 16) as zeros
     HIP_TRY(hipMemset2DAsync(e->Y + e->W, sizeof(double) * e->ld, 0, sizeof(double) * (e->ld - e->W), C.Qp, e->st));
   HIP_TRY(launch_gram(e->Y, e->ld, e->W, C.Qp, e->gpart, e->G, e->st));

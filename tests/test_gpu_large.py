@@ -100,3 +100,41 @@ def test_benzene_refresh_in_parts(Q, precision):
     el = ens.sweeps(1, 0.2, refresh_interval=0, trace=True)[3][0][some]
     ref = s.evaluate_batch(ens.positions()[some], ("eloc",))["eloc"]
     np.testing.assert_allclose(el, ref, rtol=1e-9 if precision == "fp64" else 2e-4, atol=1e-9 if precision == "fp64" else 1e-2)
+
+
+# 131,072 a part; the kernel AUTO takes depends on the call's size and not on a
+# part's (77 mixed CH4 configurations alone would go to the FP64 lane groups)
+@pytest.mark.parametrize("name,precision", [("h2", "fp64"), ("ch4", "mixed")])
+def test_derivatives_in_parts(Q, name, precision):
+    """A call past the size of one part equals, to the bit, two calls that
+    share its configurations and lie within one part."""
+    s = _system(Q, name, precision)
+    W, rng = 131072 + 77, np.random.default_rng(4)
+    pos = s.get_nuclei()[np.arange(s.n_elec) % s.n_nuc] + 0.7 * rng.normal(size=(W, s.n_elec, 3))
+    out = s.derivatives_batch(pos)
+    for a, b in ((0, 100_000), (100_000, W)):
+        ref = s.derivatives_batch(pos[a:b])
+        for k in ref:
+            np.testing.assert_array_equal(out[k][a:b], ref[k], err_msg=k)
+
+
+# host calls of up to 2 MiB share one allocation, inputs or outputs of up to 1 MiB
+# one copy each way, and derivatives of up to 128 KiB of features are unpacked on
+# the host: W on both sides of each for CH4 (240 + 416 bytes, 48 features) and H2
+# (48 + 88 bytes, 16 features, no parameters)
+@pytest.mark.parametrize("name,W", [("ch4", 341), ("ch4", 342), ("ch4", 2520), ("ch4", 2600), ("ch4", 3196), ("ch4", 3197),
+                                    ("ch4", 4369), ("ch4", 4370), ("h2", 1024), ("h2", 1025), ("h2", 15_420),
+                                    ("h2", 15_421), ("h2", 21_846)])
+def test_host_calls_around_the_copy_limits(Q, name, W):
+    """Whatever way the arrays take, the results are those of batches of 100
+    (which share one allocation and one copy each way), to the bit: the same
+    kernel runs on both."""
+    s = _system(Q, name, "fp64")
+    rng = np.random.default_rng(W)
+    pos = s.get_nuclei()[np.arange(s.n_elec) % s.n_nuc] + 0.7 * rng.normal(size=(W, s.n_elec, 3))
+    for f in (s.evaluate_batch, s.derivatives_batch):
+        out = f(pos)
+        for a in (0, W // 2, W - 100):
+            ref = f(pos[a : a + 100])
+            for k in ref:
+                np.testing.assert_array_equal(out[k][a : a + 100], ref[k], err_msg=k)
