@@ -887,7 +887,7 @@ class CallBuffers {
       return QMC_OK;
     }
     for (int i = 0; i < n_; ++i)
-      if (b_[i].out && b_[i].dev != b_[i].out)
+      if (b_[i].out && b_[i].bytes && b_[i].dev != b_[i].out)
         HIP_TRY(hipMemcpyAsync(b_[i].out, b_[i].dev, b_[i].bytes, hipMemcpyDeviceToHost, st_));
     HIP_TRY(hipMemcpyAsync(flag, flag_ptr(), sizeof(int), hipMemcpyDeviceToHost, st_));
     HIP_TRY(hipStreamSynchronize(st_));
