@@ -1,5 +1,6 @@
-"""Benzene's SR-gradient and force path on the GPU (the wave derivative
-kernel: one wavefront per walker).
+"""Benzene's SR-gradient and force path on the GPU: the kernel with one
+electron per lane that AUTO takes, and the wave derivative kernel (one
+wavefront per walker).
 
 BenzeneGTO::set_nuclei rebuilds the C-H sigma MO coefficients from the
 bond directions (benzene.rs:786-809), so the nuclear gradient Omega of
@@ -44,9 +45,11 @@ def _configs(o, W, seed=4):
     return pos
 
 
+@pytest.mark.parametrize("engine", ["auto", "wave"])
 @pytest.mark.parametrize("bent", [False, True])
-def test_benzene_derivatives_parity_fp64(Q, oracle, bent):
+def test_benzene_derivatives_parity_fp64(Q, oracle, bent, engine):
     g, o = _pair(Q, oracle, bent=bent)
+    g.set_engine(engine)
     W = 6
     pos = _configs(o, W)
     out = g.derivatives_batch(pos)
@@ -90,10 +93,17 @@ def test_benzene_omega_without_the_mo_rule_misses_the_bond_term(Q, oracle):
 
 
 def test_benzene_derivatives_mixed_precision(Q, oracle):
+    """The wave kernel's FP32 terms against FP64; under AUTO both precisions
+    run the same FP64 kernel."""
     g64, o = _pair(Q, oracle)
     g32, _ = _pair(Q, oracle, precision="mixed")
     pos = _configs(o, 8, seed=5)
-    a, b = g32.derivatives_batch(pos), g64.derivatives_batch(pos)
+    auto, b = g32.derivatives_batch(pos), g64.derivatives_batch(pos)
+    for k in b:
+        assert np.array_equal(auto[k], b[k]), k
+    g32.set_engine("wave")
+    a = g32.derivatives_batch(pos)
+    assert not np.array_equal(a["eloc"], b["eloc"])
     for k, tol in (("O", 1e-4), ("F", 1e-4), ("Om", 1e-3), ("dE", 1e-3)):
         s = np.abs(b[k]).max()
         assert np.abs(a[k] - b[k]).max() <= tol * s, (k, np.abs(a[k] - b[k]).max() / s)
@@ -110,6 +120,7 @@ def test_wave_derivatives_match_register_kernels(Q, oracle, name):
         mk = lambda: Q.MethaneGTO(1.5, 2.0, 2.06, "STO-3G", 0)
         o = oracle.System.methane_sto3g(1.5, 2.0, 2.06, 0)
     reg, wav = mk(), mk()
+    reg.set_engine("register")  # AUTO takes the lane groups for so few
     wav.set_engine("wave")
     pos = _configs(o, 40, seed=2)
     a, b = wav.derivatives_batch(pos), reg.derivatives_batch(pos)

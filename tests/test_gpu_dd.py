@@ -6,7 +6,7 @@ import math
 import numpy as np
 import pytest
 
-from test_gpu_parity import _close, _pair
+from test_gpu_parity import ENGINES, _close, _pair
 
 pytestmark = pytest.mark.gpu
 
@@ -18,12 +18,14 @@ def Q():
     return Q
 
 
+@pytest.mark.parametrize("engine", ENGINES)
 @pytest.mark.parametrize("name", ["h2", "li_ref", "li_seeded", "ch4_sto3g", "ch4_631g"])
-def test_dd_trajectory_parity_fp64(Q, oracle, name):
+def test_dd_trajectory_parity_fp64(Q, oracle, name, engine):
     """Same seed -> the Langevin single-electron moves (Sherman-Morrison
     ratio, drift from the inverse column) follow the oracle's chain step for
     step: identical decisions, positions and E_L."""
     g, o = _pair(Q, oracle, name)
+    g.set_engine(engine)
     W, steps, seed, tau = 65, 4, 21, 0.05
     ens = Q.Ensemble(g, W, seed)
     p0 = ens.positions()
@@ -35,10 +37,12 @@ def test_dd_trajectory_parity_fp64(Q, oracle, name):
     assert _close(tr, el_o, 1e-9)
 
 
-def test_dd_large_step_and_drift_cap(Q, oracle):
+@pytest.mark.parametrize("engine", ENGINES)
+def test_dd_large_step_and_drift_cap(Q, oracle, engine):
     """A time step large enough that tau F often exceeds max_drift (0.3) on
     CH4: the capped drift of vmc.rs:313-321 in both Green's functions."""
     g, o = _pair(Q, oracle, "ch4_sto3g")
+    g.set_engine(engine)
     W, steps, seed, tau, cap = 40, 3, 4, 0.4, 0.3
     ens = Q.Ensemble(g, W, seed)
     p0 = ens.positions()
@@ -49,10 +53,11 @@ def test_dd_large_step_and_drift_cap(Q, oracle):
     assert _close(tr, el_o, 1e-9)
 
 
-def test_dd_generic_kernels_match(Q, oracle):
+@pytest.mark.parametrize("engine", ENGINES)
+def test_dd_generic_kernels_match(Q, oracle, engine):
     g, o = _pair(Q, oracle, "ch4_631g")
     out = []
-    for eng in ("auto", "generic"):
+    for eng in (engine, "generic"):
         g.set_engine(eng)
         ens = Q.Ensemble(g, 70, 2)
         es, e2, acc = ens.sweeps(3, 0.03, Q.QMC_MOVE_DRIFT, refresh_interval=2, max_drift=1.0)
@@ -93,11 +98,13 @@ def test_ddvmc_run_matches_metropolis_vmc(Q):
     assert abs(r.energy - rv.energy) < 3 * math.hypot(r.error, rv.error) + 2e-4
 
 
-def test_dd_wave_benzene_trajectory_fp64(Q, oracle):
-    """Benzene's drift-diffusion moves on the wave engine follow the
-    oracle's chain in the log domain (the reference's 1e-30 guard on the
+@pytest.mark.parametrize("engine", ["auto", "wave"])
+def test_dd_wave_benzene_trajectory_fp64(Q, oracle, engine):
+    """Benzene's drift-diffusion moves on the wave engine, and on the
+    half-wave engine that AUTO takes, follow the oracle's chain in the log domain (the reference's 1e-30 guard on the
     linear psi, vmc.rs:363, rejects every benzene move: psi ~ e^-650)."""
     g = Q.BenzeneGTO(1.5, 2.0, 2.64, 2.05)
+    g.set_engine(engine)
     o = oracle.System.benzene(1.5, 2.0, 2.64, 2.05)
     W, steps, seed, tau = 3, 2, 7, 0.02
     ens = Q.Ensemble(g, W, seed)
@@ -113,7 +120,7 @@ def test_dd_wave_benzene_trajectory_fp64(Q, oracle):
 @pytest.mark.parametrize("name", ["h2", "li_seeded", "ch4_sto3g"])
 def test_dd_wave_engine_matches_register_engine(Q, oracle, name):
     out = []
-    for eng in ("auto", "wave"):
+    for eng in ("register", "wave"):
         g, _ = _pair(Q, oracle, name)
         g.set_engine(eng)
         ens = Q.Ensemble(g, 48, 5)
@@ -152,6 +159,7 @@ def test_dd_tile_engine_benzene_fp64_vs_oracle(Q, oracle):
     and E_L to 1e-9.  17 walkers make a full tile and a ragged one."""
     g = Q.BenzeneGTO(1.5, 2.0, 2.64, 2.05, precision="fp64")
     assert g.engine_name() == "tile"
+    g.set_engine("tile")  # AUTO takes the half-wave engine, tested above
     o = oracle.System.benzene(1.5, 2.0, 2.64, 2.05)
     W, steps, seed, tau = 17, 2, 7, 0.02
     ens = Q.Ensemble(g, W, seed)

@@ -22,9 +22,11 @@ def _close(a, b, rtol, scale=None):
     return np.all(np.abs(a - b) <= rtol * np.maximum(s, 1e-300) + rtol * 1e-3)
 
 
+@pytest.mark.parametrize("engine", ["auto", "wave"])  # AUTO: one electron per lane
 @pytest.mark.parametrize("ch", [2.042, 2.05])
-def test_benzene_eval_parity_fp64(Q, oracle, ch):
+def test_benzene_eval_parity_fp64(Q, oracle, ch, engine):
     g = Q.BenzeneGTO(1.5, 2.0, 2.64, ch)
+    g.set_engine(engine)
     o = oracle.System.benzene(1.5, 2.0, 2.64, ch)
     assert g.nuclear_repulsion() == pytest.approx(o.nuclear_repulsion(), rel=1e-14)
     pos = o.initialize_batch(2, 12)
@@ -39,8 +41,11 @@ def test_benzene_eval_parity_fp64(Q, oracle, ch):
     assert _close(out["eloc"], ref["eloc"], 1e-10)
 
 
-def test_benzene_mixed_precision_error(Q, oracle):
+@pytest.mark.parametrize("engine", ["auto", "wave"])
+def test_benzene_mixed_precision_error(Q, oracle, engine):
+    """The wave engine's FP32 terms; AUTO evaluates in FP64."""
     g = Q.BenzeneGTO(1.5, 2.0, 2.64, 2.05, precision="mixed")
+    g.set_engine(engine)
     o = oracle.System.benzene(1.5, 2.0, 2.64, 2.05)
     pos = o.initialize_batch(5, 8)
     ref = o.batch_eval(pos)
@@ -48,10 +53,14 @@ def test_benzene_mixed_precision_error(Q, oracle):
     assert _close(out["logabs"], ref["logabs"], 1e-12)
     err = np.abs(out["eloc"] - ref["eloc"])
     assert np.all(err <= 2e-4 * np.abs(ref["eloc"]) + 1e-2), err.max()
+    if engine == "auto":
+        assert _close(out["eloc"], ref["eloc"], 1e-10)
 
 
-def test_benzene_trajectory_parity(Q, oracle):
+@pytest.mark.parametrize("engine", ["auto", "wave"])  # AUTO: a walker on half a wavefront
+def test_benzene_trajectory_parity(Q, oracle, engine):
     g = Q.BenzeneGTO(1.5, 2.0, 2.64, 2.05)
+    g.set_engine(engine)
     o = oracle.System.benzene(1.5, 2.0, 2.64, 2.05)
     W, steps, seed, step = 3, 2, 7, 0.2
     ens = Q.Ensemble(g, W, seed)
@@ -68,6 +77,7 @@ def test_wave_engine_matches_register_engine(Q, oracle, name):
     from test_gpu_parity import _configs, _pair
     g, o = _pair(Q, oracle, name)
     pos = _configs(o, 40)
+    g.set_engine("register")
     reg = g.evaluate_batch(pos)
     g.set_engine("wave")
     wav = g.evaluate_batch(pos)
