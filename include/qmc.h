@@ -184,13 +184,25 @@ int qmc_set_precision(qmc_system* sys, int32_t precision);
  * engine moves 16 walkers per workgroup together with an MFMA MO
  * contraction (sweeps of 21 + 21-electron systems such as benzene).  AUTO
  * picks the register engine when it exists for the system, else the tile
- * engine when it fits, else the wave engine.  Under AUTO, FP64 work of few
- * walkers of a compiled shell structure runs one electron per lane, and FP64
- * benzene sweeps run with a walker on half a wavefront; evaluations and
- * derivatives of benzene run one electron per lane unless WAVE is selected.
- * The register engine uses kernels specialised to the system's
- * shell structure when one is compiled (H2, both Li atoms, CH4 STO-3G and
- * 6-31G); GENERIC forces its kernels with run-time shell loops. */
+ * engine when it fits, else the wave engine.
+ *  - The register engine uses kernels specialised to the system's shell
+ *    structure when one is compiled (H2, both Li atoms, CH4 STO-3G and
+ *    6-31G); GENERIC forces its kernels with run-time shell loops.
+ *  - All-electron moves of the register engine's electron counts run one
+ *    electron per lane, for any number of walkers and under AUTO, REGISTER
+ *    and GENERIC, with energies in FP64 in both precisions.
+ *  - Under AUTO, calls with few walkers of a compiled structure without Pade
+ *    series terms run one electron per lane in FP64: FP64 sweeps up to
+ *    16,384 walkers (CH4, Li) or 32,768 (H2); and, in both precisions,
+ *    evaluations up to 32,768 (CH4) or 65,536 (H2, Li) configurations and
+ *    derivatives and samples up to 8,192 (CH4) or 16,384 (Li).  A MIXED
+ *    system's evaluations and derivatives are therefore FP64-accurate up to
+ *    that size of the call and run in FP32 above it; select REGISTER for
+ *    FP32 at every size.  FP64 results on the two sides differ by rounding.
+ *  - 21 + 21-electron systems without series terms: under AUTO, FP64 sweeps
+ *    run with a walker on half a wavefront; evaluations, derivatives and
+ *    samples run one electron per lane in FP64, in both precisions and for
+ *    any number of walkers, unless WAVE is selected. */
 #define QMC_ENGINE_AUTO 0
 #define QMC_ENGINE_REGISTER 1
 #define QMC_ENGINE_WAVE 2
@@ -199,9 +211,9 @@ int qmc_set_precision(qmc_system* sys, int32_t precision);
 int qmc_set_engine(qmc_system* sys, int32_t engine);
 /* Name of the engine a system's sweeps run on: "tile", "wave",
  * "register/generic" or "register/<shell structure>" (no reference
- * counterpart; diagnostics).  Under AUTO, FP64 sweeps of a "tile" system and
- * FP64 sweeps of few walkers of a "register" one run on that engine's
- * kernels with more lanes per walker (32, and one per electron). */
+ * counterpart; diagnostics).  It does not tell the kernels that AUTO takes
+ * by the precision and the number of walkers: one electron per lane for a
+ * "register" system, half a wavefront per walker for a "tile" one (above). */
 int qmc_engine_name(const qmc_system* sys, char* buf, int32_t len);
 int qmc_set_flags(qmc_system* sys, uint32_t flags);
 int qmc_system_info(const qmc_system* sys, int32_t* n_elec, int32_t* n_up, int32_t* n_nuc, int32_t* n_ao);
@@ -295,7 +307,9 @@ typedef struct {
   int32_t n_steps;          /* sweeps to run */
   double step_size;         /* Gaussian proposal width (bohr), or the time step tau of QMC_MOVE_DRIFT */
   int32_t refresh_interval; /* FP64 inverse refresh every this many sweeps (0: never) */
-  int32_t steps_per_launch; /* sweeps per persistent launch (0: library default) */
+  int32_t steps_per_launch; /* sweeps per persistent launch (0: library default); fewer where their
+                               partial sums would take more than 32 MiB and the memory that 64
+                               walkers per partial sum need */
   double max_drift;         /* QMC_MOVE_DRIFT: cap of |tau F| per electron (vmc.rs:313-321) */
 } qmc_sweep_params;
 

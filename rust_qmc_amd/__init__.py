@@ -155,7 +155,7 @@ class System:
         check(lib().qmc_set_engine(self._h, {"auto": 0, "register": 1, "wave": 2, "generic": 3, "tile": 4}[engine]))
 
     def engine_name(self):
-        """The kernels this system runs on, e.g. 'register/ch4-sto3g'."""
+        """The engine this system's sweeps run on, e.g. 'register/ch4-sto3g'."""
         buf = C.create_string_buffer(64)
         check(lib().qmc_engine_name(self._h, buf, 64))
         return buf.value.decode()

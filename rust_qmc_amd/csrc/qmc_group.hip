@@ -20,8 +20,14 @@ namespace qmc {
 // its sector's inverse, and a launch has G times the wavefronts.  Measured in
 // FP64, us per step, before / now: H2 7.6 / 3.1 at 20 walkers and 8.7 / 5.3
 // at 65,536; Li 22 / 5.0 at 16,384; CH4 STO-3G 137 / 18 at 8,192, 148 / 129
-// at 65,536; CH4 6-31G 203 / 145 at 65,536.  Bound by the latency of the
-// chain (dependent FP64 instructions) up to one wavefront per SIMD.
+// at 65,536; CH4 6-31G 203 / 145 at 65,536.  Up to one
+// wavefront per SIMD a step takes the time of one wavefront's own
+// instructions: 66 % of its cycles issue vector instructions (970 a step for
+// H2 at 4,096 walkers, 3,270 for CH4 6-31G at 20), 20 to 22 % wait for LDS,
+// scalar loads and permutes, the rest are dependences.  The compiled CH4
+// instances take 256 vector registers and 63 to 186 accumulator ones as
+// overflow, and keep 260 to 380 scalar values in vector lanes (6-31G most);
+// no instance uses scratch.
 // ---------------------------------------------------------------------------
 template <int NU, int ND, class Bs, class Js, class T>
 __global__ void __launch_bounds__(64) group_ae_kernel(const DevSys<double>* __restrict__ Sp, EnsView<T> E,

@@ -15,6 +15,11 @@
 //     the Sherman-Morrison update of the lane's own column.
 // Wavefronts never wait for each other: the MFMA tile that this replaces
 // spent two workgroup barriers per move and held one wavefront per SIMD.
+// In drift-diffusion sweeps of 2,048 walkers, one wavefront per SIMD, a
+// wavefront waits 46 % of its cycles (LDS reads above all) and issues vector
+// instructions for 40 %; in Metropolis sweeps of 8,192, two per SIMD, 49 % and
+// 27 %.  A drift-diffusion sweep is 64,900 vector and 9,000 LDS instructions,
+// whose bank conflicts hold the LDS for 13 % of the time.
 #include "qmc_half.hpp"
 
 #include "qmc_terms_dev.hpp"
@@ -436,7 +441,7 @@ hipError_t launch_by_count(const void* Sd, const TermTab* T, EnsView<double> E, 
                            double* trace, hipStream_t st) {
   // Up to 2,048 walkers one wavefront per SIMD covers the chip, with 512
   // registers each; past that two per SIMD share a CU's tables, at 256
-  // registers (some spill).  us per sweep, four / eight wavefronts per
+  // registers (53 and 77 of them spilled to scratch).  us per sweep, four / eight wavefronts per
   // workgroup / the tile engine: Metropolis 202 / 275 / 371 at 2,048 walkers,
   // 393 / 277 / 373 at 4,096, 782 / 550 / 742 at 8,192; drift-diffusion 290 /
   // 445 / 569, 576 / 448 / 570, 1,146 / 894 / 1,137.

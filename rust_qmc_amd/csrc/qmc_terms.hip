@@ -12,9 +12,12 @@
 // with a wavefront per walker, about 350 here; 1,003 evaluations 458 -> 105
 // us a call.  Cycles per wavefront: Slater rows 50 k, inversion 41 k,
 // determinant and nuclear terms 80 k, partners 11 k, parameters 20 k, for
-// about 10 k instructions: the latency of scalar loads (coefficient rows) and
-// of dependent FP64 instructions is what counts.  The rows from LDS were
-// slower (500 us a measure call against 402: the wider loads spill).
+// about 20 k vector and 1 k scalar-load instructions: a wavefront waits 39 %
+// of its cycles (coefficient rows from the scalar cache, rows in transit) and
+// issues vector instructions for 33 %, at two wavefronts per SIMD (1,003
+// evaluations, under one per SIMD: 51 % and 32 %).  The rows from LDS were
+// slower (500 us a measure call against 402: the wider loads spill).  The
+// evaluation spills 24 registers (100 bytes of scratch), the derivatives none.
 #include "qmc_terms.hpp"
 
 #include <cstring>
