@@ -300,7 +300,7 @@ int qmc_ensemble_refresh(qmc_ensemble* ens);
 #define QMC_MOVE_SINGLE 0 /* single-electron Gaussian moves, Sherman-Morrison */
 #define QMC_MOVE_ALL 1    /* all-electron moves, MCMCSimulation::metropolis_step (vmc.rs:95-119) */
 #define QMC_MOVE_DRIFT 2  /* drift-diffusion single-electron moves, DriftDiffusionVMC::sweep
-                             (vmc.rs:382-438); register engine */
+                             (vmc.rs:382-438) */
 
 typedef struct {
   int32_t move;             /* QMC_MOVE_* */
